@@ -418,11 +418,10 @@ typedef struct vg_nav_states {
 
 /* Navigator selection (navigation/SimpleNavigator.h:341-482,
  * navigation/ABBoxNavigator.h:201-424).  VG_NAV_ABBOX_MIXED is the ABBox
- * navigator with an FP32 filter in its daughter walk: a daughter whose FP32
- * lower bound on the distance from the point (with a rigorous rounding
- * margin) exceeds the best step found so far is not evaluated in FP64.  Its
- * steps, next volumes and states are those of VG_NAV_ABBOX, bit for bit; no
- * counterpart in the reference. */
+ * navigator with its daughters preselected in FP32.  VG_NAV_ABBOX now does
+ * the same (an index over each volume's daughters, with a rounding margin,
+ * says which of them a step can meet), so both names select one navigator;
+ * steps, next volumes and states are those of a walk over every daughter. */
 #define VG_NAV_ABBOX 0
 #define VG_NAV_SIMPLE 1
 #define VG_NAV_ABBOX_MIXED 2

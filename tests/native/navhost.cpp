@@ -22,7 +22,6 @@ constexpr int kExactOnlyKind = 9;
 
 struct HostGeom {
   vg_geometry g;
-  std::vector<float> aabbf;
   NavDev dev;
 };
 
@@ -63,7 +62,8 @@ void Locate(const HostGeom *h, long n, const double *x, const double *y, const d
     for (long i = b; i < e; ++i) {
       DPath<D> p;
       p.Clear();
-      LocatePoint(h->dev, h->dev.world, V3{x[i], y[i], z[i]}, p, true);
+      const Target t = FromWorld<D, kAllShapes>(h->dev, V3{x[i], y[i], z[i]}, p);
+      Descend<D, kAllShapes>(h->dev, t, p);
       Store(p, depth, n, i, level, path);
     }
   });
@@ -75,27 +75,21 @@ void Step(const HostGeom *h, long n, const double *x, const double *y, const dou
           int *path_out, unsigned char *boundary_out, double *step_out, double pstep, int kind, int nthreads) {
   ParallelFor(n, nthreads, [&](long b, long e) {
     for (long i = b; i < e; ++i) {
-      DPath<D> c, o;
-      Load(level_in, path_in, n, i, c);
+      DPath<D> o;
+      Load(level_in, path_in, n, i, o);
       double step = 0;
+      const V3 q{x[i], y[i], z[i]}, v{dx[i], dy[i], dz[i]};
       if (kind == VG_NAV_SIMPLE_BASKET) {
         DPath<D> c0;
         Load(level_in, path_in, n, 0, c0);
-        if (c.level > 0 && c0.level > 0)
-          FindNextBoundaryAndStepBasket(h->dev, V3{x[i], y[i], z[i]}, V3{dx[i], dy[i], dz[i]}, c, o, pstep, step,
-                                        c0.Top());
-        else
-          o = c;
-      } else if (c.level > 0 && kind == kExactOnlyKind) {
-        FindNextBoundaryAndStep<D, true>(h->dev, V3{x[i], y[i], z[i]}, V3{dx[i], dy[i], dz[i]}, c, o, pstep, step,
-                                         VG_NAV_ABBOX);
-      } else if (c.level > 0 && kind == VG_NAV_ABBOX_MIXED) {
-        FindNextBoundaryAndStep<D, false, kAllShapes, true>(h->dev, V3{x[i], y[i], z[i]}, V3{dx[i], dy[i], dz[i]}, c,
-                                                            o, pstep, step, kind);
-      } else if (c.level > 0) {
-        FindNextBoundaryAndStep(h->dev, V3{x[i], y[i], z[i]}, V3{dx[i], dy[i], dz[i]}, c, o, pstep, step, kind);
-      } else {
-        o = c;
+        if (o.level > 0 && c0.level > 0)
+          FindNextBoundaryAndStep<D, kAllShapes, kWayBasket>(h->dev, q, v, o, pstep, step, c0.Top());
+      } else if (o.level > 0 && kind == kExactOnlyKind) {
+        FindNextBoundaryAndStep<D, kAllShapes, kWayAbboxSorted>(h->dev, q, v, o, pstep, step, o.Top());
+      } else if (o.level > 0 && kind == VG_NAV_SIMPLE) {
+        FindNextBoundaryAndStep<D, kAllShapes, kWaySimple>(h->dev, q, v, o, pstep, step, o.Top());
+      } else if (o.level > 0) {
+        FindNextBoundaryAndStep<D, kAllShapes, kWayAbbox>(h->dev, q, v, o, pstep, step, o.Top());
       }
       Store(o, depth, n, i, level_out, path_out);
       boundary_out[i] = (unsigned char)o.boundary;
@@ -111,7 +105,7 @@ void Safety(const HostGeom *h, long n, const double *x, const double *y, const d
     for (long i = b; i < e; ++i) {
       DPath<D> c;
       Load(level_in, path_in, n, i, c);
-      out[i] = c.level > 0 ? GetSafety(h->dev, V3{x[i], y[i], z[i]}, c) : 0.;
+      out[i] = c.level > 0 ? GetSafety<D, kAllShapes>(h->dev, V3{x[i], y[i], z[i]}, c) : 0.;
     }
   });
 }
@@ -128,10 +122,10 @@ void Trace(const HostGeom *h, long n, const double *x, const double *y, const do
       int nexact;
       const V3 dd{dx[i], dy[i], dz[i]};
       nsteps[i] = kind == kExactOnlyKind
-                      ? TraceOne<D, true>(h->dev, p, dd, pstep, VG_NAV_ABBOX, max_steps, dist, hh, nexact)
-                  : kind == VG_NAV_ABBOX_MIXED
-                      ? TraceOne<D, false, kAllShapes, true>(h->dev, p, dd, pstep, kind, max_steps, dist, hh, nexact)
-                      : TraceOne<D>(h->dev, p, dd, pstep, kind, max_steps, dist, hh, nexact);
+                      ? TraceOne<D, kAllShapes, kWayAbboxSorted>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact)
+                  : kind == VG_NAV_SIMPLE
+                      ? TraceOne<D, kAllShapes, kWaySimple>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact)
+                      : TraceOne<D, kAllShapes, kWayAbbox>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact);
       fx[i] = p.x;
       fy[i] = p.y;
       fz[i] = p.z;
@@ -156,18 +150,17 @@ void *navhost_geom_create(int n_shapes, const int *shape_type, const int *shape_
     delete h;
     return nullptr;
   }
-  h->aabbf.assign(h->g.aabb.begin(), h->g.aabb.end());
+  h->dev.nav = h->g.nav.data();
   h->dev.placed = h->g.placed.data();
   h->dev.params = h->g.params.data();
-  h->dev.daughters = h->g.daughters.data();
-  h->dev.aabb = h->aabbf.data();
-  h->dev.b32 = h->g.b32.data();
-  h->dev.b32side = h->g.b32side.data();
   h->dev.slot_box = h->g.slot_aabb.data();
+  h->dev.dindex = h->g.dindex.data();
+  h->dev.dmasks = h->g.dmasks.data();
   h->dev.world = h->g.world;
   h->dev.n_placed = (int32_t)h->g.placed.size();
   h->dev.n_daughters = (int32_t)h->g.daughters.size();
-  h->dev.pad = 0;
+  h->dev.n_index = (int32_t)h->g.dindex.size();
+  h->dev.n_masks = (int32_t)h->g.dmasks.size();
   return h;
 }
 
@@ -214,9 +207,9 @@ int navhost_query(void *hv, int pv, int query, long n, const double *x, const do
                   const double *dx, const double *dy, const double *dz, const double *sm, void *out) {
   auto *h = static_cast<HostGeom *>(hv);
   const NavDev &g = h->dev;
-  const PlacedRec &r = g.Pv(pv);
-  Xf xf;
-  LoadXf(r, xf);
+  VGA_NAV_CHECK(pv >= 0 && pv < g.n_placed, "placed id out of range");
+  const PlacedRec &r = g.placed[pv];
+  const Xf xf = r.xf;
   const double *blk = g.params + r.param_off;
   for (long i = 0; i < n; ++i) {
     const V3 p{x[i], y[i], z[i]};

@@ -31,13 +31,17 @@ namespace {
 void FreeDevice(vg_geometry *g) {
   if (g->d_params) (void)hipFree(g->d_params);
   if (g->d_placed) (void)hipFree(g->d_placed);
-  if (g->d_daughters) (void)hipFree(g->d_daughters);
-  if (g->d_aabb) (void)hipFree(g->d_aabb);
   if (g->d_b32) (void)hipFree(g->d_b32);
   if (g->d_b32side) (void)hipFree(g->d_b32side);
   if (g->d_extent32) (void)hipFree(g->d_extent32);
   if (g->d_slot_aabb) (void)hipFree(g->d_slot_aabb);
+  if (g->d_nav) (void)hipFree(g->d_nav);
+  if (g->d_dindex) (void)hipFree(g->d_dindex);
+  if (g->d_dmasks) (void)hipFree(g->d_dmasks);
   if (g->d_scalar) (void)hipFree(g->d_scalar);
+  g->d_nav = nullptr;
+  g->d_dindex = nullptr;
+  g->d_dmasks = nullptr;
   g->d_slot_aabb = nullptr;
   g->d_scalar = nullptr;
   g->d_b32 = nullptr;
@@ -45,8 +49,6 @@ void FreeDevice(vg_geometry *g) {
   g->d_extent32 = nullptr;
   g->d_params = nullptr;
   g->d_placed = nullptr;
-  g->d_daughters = nullptr;
-  g->d_aabb = nullptr;
 }
 
 template <class T>
@@ -107,15 +109,15 @@ int vg_geometry_upload(const vg_flat_geometry *f, vg_geometry **out) {
     return rc;
   }
   // Device copies.
-  std::vector<float> faabb(g->aabb.begin(), g->aabb.end());
   rc = Upload(g->params, &g->d_params);
   if (!rc) rc = Upload(g->placed, &g->d_placed);
-  if (!rc) rc = Upload(g->daughters, &g->d_daughters);
-  if (!rc) rc = Upload(faabb, &g->d_aabb);
   if (!rc) rc = Upload(g->b32, &g->d_b32);
   if (!rc) rc = Upload(g->b32side, &g->d_b32side);
   if (!rc) rc = Upload(g->extent32, &g->d_extent32);
   if (!rc) rc = Upload(g->slot_aabb, &g->d_slot_aabb);
+  if (!rc) rc = Upload(g->nav, &g->d_nav);
+  if (!rc) rc = Upload(g->dindex, &g->d_dindex);
+  if (!rc) rc = Upload(g->dmasks, &g->d_dmasks);
   if (!rc) rc = Upload(std::vector<double>(16, 0.), &g->d_scalar);
   if (rc) {
     FreeDevice(g);

@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "shapes.hpp"
 #include "vg_internal.hpp"
 
 namespace vga {
@@ -82,6 +83,126 @@ void ComputeAABB(const double lo[3], const double hi[3], const Xf &X, double *ou
   for (int r = 0; r < 3; ++r) {
     out6[r] = mn[r] - 1E-3;
     out6[3 + r] = mx[r] + 1E-3;
+  }
+}
+
+// A rotation whose rows are unit vectors at right angles.
+bool Orthonormal(const Xf &X) {
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j <= i; ++j) {
+      double s = 0;
+      for (int k = 0; k < 3; ++k) s += X.r[3 * i + k] * X.r[3 * j + k];
+      if (!(std::fabs(s - (i == j ? 1. : 0.)) < 1e-9)) return false;
+    }
+  return true;
+}
+
+bool Bits(double a, double b) { return std::memcmp(&a, &b, sizeof a) == 0; }
+
+// The navigator's record of a placed volume.  A placement that is no exact
+// translation or rotation about z keeps its full matrix; a matrix that is
+// one is restored bit for bit from the numbers kept.
+NavRec MakeNavRec(const PlacedRec &r, const double *blk) {
+  NavRec n{};
+  n.index = -1;
+  n.dbegin = r.dbegin;
+  n.nd = r.dend - r.dbegin;
+  n.type = r.type;
+  n.param_off = r.param_off;
+  n.code = kFormGeneral;
+  switch (r.type) {
+    case VG_BOX: {
+      const BoxP &b = *reinterpret_cast<const BoxP *>(blk);
+      n.code = kFormBox;
+      for (int i = 0; i < 3; ++i) n.s[i] = b.d[i];
+      break;
+    }
+    case VG_TUBE: {
+      const TubeP &t = *reinterpret_cast<const TubeP *>(blk);
+      if (t.hasPhi != 0) break;
+      n.code = kFormTube;
+      n.s[0] = t.rmin;
+      n.s[1] = t.rmax;
+      n.s[2] = t.z;
+      break;
+    }
+    case VG_TRD: {
+      const TrdP &t = *reinterpret_cast<const TrdP *>(blk);
+      n.code = kFormTrd;
+      n.s[0] = t.dx1;
+      n.s[1] = t.dx2;
+      n.s[2] = t.dy1;
+      n.s[3] = t.dy2;
+      n.s[4] = t.dz;
+      n.s[5] = t.fx;
+      break;
+    }
+    case VG_ORB: {
+      const OrbP &o = *reinterpret_cast<const OrbP *>(blk);
+      n.code = kFormOrb;
+      n.s[0] = o.r;
+      n.s[1] = o.rTolI;
+      n.s[2] = o.rTolO;
+      break;
+    }
+  }
+  n.code |= r.xfkind << kNavKindShift;
+  const double *m = r.xf.r;
+  bool about_z = Bits(m[8], 1.);
+  for (int i : {2, 5, 6, 7}) about_z &= Bits(m[i], 0.);
+  const bool unit = about_z && Bits(m[0], 1.) && Bits(m[1], 0.) && Bits(m[3], 0.) && Bits(m[4], 1.);
+  const bool still = Bits(r.xf.t[0], 0.) && Bits(r.xf.t[1], 0.) && Bits(r.xf.t[2], 0.);
+  if (!about_z) {
+    n.code |= kNavMatrix;
+    return n;
+  }
+  if (!still) n.code |= kNavMoves;
+  if (!unit) n.code |= kNavTurns;
+  for (int i = 0; i < 3; ++i) n.t[i] = r.xf.t[i];
+  n.r[0] = m[0];
+  n.r[1] = m[1];
+  n.r[2] = m[3];
+  n.r[3] = m[4];
+  return n;
+}
+
+// Daughter indexes of the logical volumes with at least kIndexMinDaughters
+// daughters.  A volume with a daughter whose matrix is no rotation gets none
+// (its extent along the mother's axes would mean nothing), and none is built
+// beyond kIndexMaxWords of masks in all.
+constexpr int kIndexMinDaughters = 3;
+constexpr size_t kIndexMaxWords = size_t(1) << 25;  // 256 MiB
+
+void BuildIndexes(vg_geometry *g) {
+  const int nl = (int)g->logical_shape.size();
+  std::vector<int32_t> of(nl, -1), axes_code(nl, 0);
+  std::vector<DaughterExtent> ext;
+  for (int l = 0; l < nl; ++l) {
+    const int db = g->logical_dbegin[l], de = g->logical_dbegin[l + 1];
+    if (de - db < kIndexMinDaughters) continue;
+    ext.clear();
+    bool ok = true;
+    for (int k = db; k < de && ok; ++k) {
+      const PlacedRec &r = g->placed[g->daughters[k]];
+      const double *blk = g->params.data() + r.param_off;
+      double lo[3], hi[3];
+      ok = Orthonormal(r.xf) && ShapeExtent(r.type, blk, lo, hi);
+      if (ok) ext.push_back(ExtentInMother(r.type, blk, r.xf, lo, hi, g->aabb.data() + 6 * (size_t)g->daughters[k]));
+    }
+    if (!ok) continue;
+    if (g->dmasks.size() + DaughterIndexWords(de - db) > kIndexMaxWords) continue;
+    of[l] = (int32_t)g->dindex.size();
+    IndexAxes axes;
+    g->dindex.push_back(BuildDaughterIndex(ext, g->dmasks, &axes));
+    axes_code[l] = axes.count << kNavAxesShift;
+    for (int a = 0; a < axes.count; ++a) axes_code[l] |= axes.coord[a] << (kNavCoordShift + 2 * a);
+  }
+  g->nav.resize(g->placed.size());
+  for (size_t p = 0; p < g->placed.size(); ++p) {
+    const PlacedRec &r = g->placed[p];
+    g->nav[p] = MakeNavRec(r, g->params.data() + r.param_off);
+    g->nav[p].code |= axes_code[r.logical];
+    g->nav[p].index = of[r.logical];
   }
 }
 
@@ -184,12 +305,18 @@ int BuildGeometry(const vg_flat_geometry *f, vg_geometry *g) {
     // Navigation and serving dispatch primitive shapes only.
     if (!g->nav_bad_type && (!ShapeHasKernels(r.type) || r.type == VG_BOOLEAN)) g->nav_bad_type = r.type;
     if (r.type >= 0 && r.type < 32) g->type_mask |= 1u << r.type;
+    if (r.type == VG_TUBE && reinterpret_cast<const TubeP *>(g->params.data() + r.param_off)->hasPhi != 0)
+      g->type_mask |= 1u;
   }
-  // The daughters' float boxes in daughter-slot order: the navigator's box
-  // loop then reads slot k's box without first reading slot k's id.
+  // The daughters' float boxes in daughter-slot order, each with the
+  // daughter's placed id: one record answers slot k's box test and says where
+  // its volume is.
   g->slot_aabb.assign(8 * g->daughters.size(), 0.f);
-  for (size_t k = 0; k < g->daughters.size(); ++k)
+  for (size_t k = 0; k < g->daughters.size(); ++k) {
     for (int i = 0; i < 6; ++i) g->slot_aabb[8 * k + i] = (float)g->aabb[6 * (size_t)g->daughters[k] + i];
+    std::memcpy(&g->slot_aabb[8 * k + 6], &g->daughters[k], sizeof(int32_t));
+  }
+  BuildIndexes(g);
   g->max_depth = Depth(g, g->world, 1, 64);
   if (g->max_depth < 0) {
     return SetError(VG_ERR_INVALID, "volume tree deeper than 64 levels or cyclic");

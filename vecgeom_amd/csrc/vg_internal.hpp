@@ -10,6 +10,7 @@
 
 #include "../../include/vecgeom_amd.h"
 #include "vg_bound32.hpp"
+#include "vg_daughter_index.hpp"
 #include "vg_math.hpp"
 
 namespace vga {
@@ -27,6 +28,32 @@ struct PlacedRec {
   Xf xf;
 };
 static_assert(sizeof(PlacedRec) % 8 == 0, "PlacedRec must be 8-byte sized");
+
+// What the navigator reads of a placed volume, in one 128-byte cache line:
+// a lane of a wave whose tracks are in different volumes gathers its record
+// alone, so the number of load instructions, not their reuse, is what the
+// record costs.  The first half holds the daughters and the parameters of
+// the simple shapes, the second the placement.
+enum NavForm : int { kFormGeneral = 0, kFormBox, kFormTube, kFormTrd, kFormOrb };
+constexpr int kNavFormMask = 7;        // NavForm; general: type and param_off
+constexpr int kNavKindShift = 3;       // XfKind of the placement (2 bits)
+constexpr int kNavMoves = 1 << 5;      // t is read
+constexpr int kNavTurns = 1 << 6;      // r is read: a rotation about z, r[0], r[1], r[3], r[4] of the matrix
+constexpr int kNavMatrix = 1 << 7;     // the placement is read from the PlacedRec
+constexpr int kNavAxesShift = 8;       // coordinates of the daughter index: count (2 bits),
+constexpr int kNavCoordShift = 10;     // then 2 bits each
+struct alignas(128) NavRec {
+  int32_t code;
+  int32_t index;   // daughter index of its logical volume (-1: none)
+  int32_t dbegin;  // first daughter slot
+  int32_t nd;      // daughters
+  double s[6];     // Box: d; Tube without phi section: rmin, rmax, z; Trd: dx1, dx2, dy1, dy2, dz, fx; Orb: r, tolerances
+  double t[3];
+  double r[4];
+  int32_t type;
+  int32_t param_off;
+};
+static_assert(sizeof(NavRec) == 128, "one cache line");
 
 struct ShapeRec {
   int32_t type;
@@ -56,20 +83,24 @@ struct vg_geometry {
   std::vector<vga::B32> b32;            // FP32 bound record per placed volume
   std::vector<float> b32side;           // variable-length bound data
   std::vector<float> extent32;          // 6 per placed: local extent lo xyz, hi xyz
-  std::vector<float> slot_aabb;         // 8 per daughter slot: its float AABB, lo xyz, hi xyz, 2 unused
+  std::vector<vga::NavRec> nav;            // per placed volume
+  std::vector<vga::DaughterIndex> dindex;  // daughter indexes (NavRec::index)
+  std::vector<uint64_t> dmasks;            // their masks
+  std::vector<float> slot_aabb;         // 8 per daughter slot: its float AABB, lo xyz, hi xyz, its placed id (int32), unused
   // Device copies.
   double *d_params = nullptr;
   vga::PlacedRec *d_placed = nullptr;
-  int32_t *d_daughters = nullptr;
-  float *d_aabb = nullptr;  // 6 floats per placed (ABBoxManager keeps floats)
   vga::B32 *d_b32 = nullptr;
   float *d_b32side = nullptr;
   float *d_extent32 = nullptr;
   float *d_slot_aabb = nullptr;
+  vga::NavRec *d_nav = nullptr;
+  vga::DaughterIndex *d_dindex = nullptr;
+  uint64_t *d_dmasks = nullptr;
   double *d_scalar = nullptr;  // device staging of vg_scalar_query (16 doubles)
   std::mutex scalar_mutex;     // one vg_scalar_query at a time per geometry
   int32_t nav_bad_type = 0;  // first shape type in the tree without device kernels (0: none)
-  uint32_t type_mask = 0;    // bit t set: some placed volume has shape type t
+  uint32_t type_mask = 0;    // bit t set: some placed volume has shape type t (bit 0: a Tube with a phi section)
 };
 
 namespace vga {

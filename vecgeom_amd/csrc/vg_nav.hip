@@ -15,25 +15,30 @@
 //   track loop                      test/globalbenchmarks/TraceTrack.cpp:170-220
 //
 // Layout and execution:
-//  * the geometry is the uploaded flat tree: PlacedRec (type, parameter
-//    offset, daughter range, placement) per placed volume, the daughter
-//    list, the shape parameter blocks, and float AABBs (6 per placed
-//    volume, in the mother frame) -- a few hundred KB for thousands of
-//    placements, resident in L2;
+//  * what bounds it: a wave's tracks are in different volumes, so each lane
+//    gathers its own volume records and the kernel lives on the texture
+//    pipe and on latency, not on HBM (100 B per track) or FP64 issue.  Each
+//    volume is therefore one 128-byte record (NavRec) of which only the
+//    parts that matter are loaded, the daughters a step can meet come from
+//    bit masks (vg_daughter_index.hpp: 1.0 box tests a step on the nested
+//    geometry instead of 47), and each kernel carries the code of one
+//    navigator and of the shapes the geometry uses.  Against full daughter
+//    scans of 128-byte placements and parameter blocks, 524,288 nested
+//    tracks went from 72.0 to 7.1 ms, 1,000 from 18.9 to 1.8 ms;
 //  * a track's path lives in registers (template depth D, unrolled selects
 //    instead of indexed private memory); the global-to-local matrix is
 //    recomputed from the path every step, as TopMatrix does;
 //  * the shape of a volume is dispatched at run time by a switch over the
-//    type tag (the reference makes a virtual call);
+//    record's form (the reference makes a virtual call);
 //  * ABBox daughter loop.  The reference sorts the boxes hit by the ray by
 //    entry distance and walks them in that order until a box starts beyond
 //    the current step.  A lane cannot hold a sorted list of up to
-//    hundreds of hits, so it first walks the daughters in index order,
-//    computing DistanceToIn for every hit box with stepMax = the initial
-//    step.  The result equals the sorted walk when (a) no hit box with a
-//    negative entry distance contains the point, (b) every DistanceToIn
-//    result is >= 0 and >= its box entry distance (boxes bound their
-//    shapes, so a box skipped by the sorted walk cannot hold a nearer
+//    hundreds of hits, so it first takes the daughters on its way in any
+//    order, computing DistanceToIn for every hit box with stepMax = the
+//    initial step.  The result equals the sorted walk when (a) no hit box
+//    with a negative entry distance contains the point, (b) every
+//    DistanceToIn result is >= 0 and >= its box entry distance (boxes bound
+//    their shapes, so a box skipped by the sorted walk cannot hold a nearer
 //    surface), and (c) the smallest distance is reached by one daughter
 //    only.  The lane checks (a)-(c) and otherwise redoes the step in exact
 //    sorted order by repeated selection of the next (distance, index) pair.
@@ -82,15 +87,30 @@ VGA_NAV void StoreState(const vg_nav_states &s, uint64_t i, const DPath<D> &p) {
   for (int l = 0; l < s.depth; ++l) s.path[(uint64_t)l * s.capacity + i] = l < D ? p.Get(l) : -1;
 }
 
+// Occupancy floors of the fused trace kernel.  Its 168 VGPRs over the basic
+// shapes hold three waves per SIMD; a fourth spills 47 registers, and the
+// spills cost more of the memory pipe (which the gathers of volume records
+// already keep busy) than the wave hides: 524,288 nested tracks 7.1 ms with
+// 3, 9.4 with 4, 16.4 with 5.  With every shape the kernel would take 330
+// registers and run one wave; two with some spills take the zoo geometry's
+// 200,001 tracks from 350 to 260 us.
+constexpr int TraceWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 3 : 2; }
+
+// The single-step kernels: with every shape two waves as above; over the
+// basic shapes the compiler's own choice (their registers hold three or
+// more).
+constexpr int StepWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 1 : 2; }
+
 template <int D, uint32_t M>
 __global__ __launch_bounds__(kNavBlock) void LocateKernel(const NavDev g, const double *__restrict__ x,
                                                           const double *__restrict__ y, const double *__restrict__ z,
-                                                          uint64_t n, const vg_nav_states s) {
-  const uint64_t i = (uint64_t)blockIdx.x * kNavBlock + threadIdx.x;
+                                                          uint64_t n, const vg_nav_states s, int shift) {
+  const uint64_t i = TrackOf((uint64_t)blockIdx.x * kNavBlock + threadIdx.x, shift, n);
   if (i >= n) return;
   DPath<D> p;
   p.Clear();
-  LocatePoint<D, M>(g, g.world, V3{x[i], y[i], z[i]}, p, true);
+  const Target t = FromWorld<D, M>(g, V3{x[i], y[i], z[i]}, p);
+  Descend<D, M>(g, t, p);
   StoreState(s, i, p);
 }
 
@@ -98,48 +118,43 @@ struct StepArgs {
   const double *x, *y, *z, *dx, *dy, *dz, *pstep;
   double *step;
   uint64_t n;
-  int32_t kind;
+  int32_t shift;  // LanesShift(n)
   int32_t pad;
 };
 
-template <int D, uint32_t M, bool MX>
-__global__ __launch_bounds__(kNavBlock) void StepKernel(const NavDev g, const StepArgs a, const vg_nav_states cur,
-                                                        const vg_nav_states nxt) {
-  const uint64_t i = (uint64_t)blockIdx.x * kNavBlock + threadIdx.x;
+template <int D, uint32_t M, int Way>
+__global__ __launch_bounds__(kNavBlock) __attribute__((amdgpu_waves_per_eu(StepWaves(M)))) void StepKernel(
+    const NavDev g, const StepArgs a, const vg_nav_states cur, const vg_nav_states nxt) {
+  const uint64_t i = TrackOf((uint64_t)blockIdx.x * kNavBlock + threadIdx.x, a.shift, a.n);
   if (i >= a.n) return;
-  DPath<D> c, o;
-  LoadState(cur, i, c);
+  DPath<D> o;
+  LoadState(cur, i, o);
   double step = 0;
   const double ps = a.pstep ? a.pstep[i] : kInfinity;
-  if (a.kind == VG_NAV_SIMPLE_BASKET) {
+  bool valid = ValidState(g, o);
+  int vol = o.Top();
+  if constexpr (Way == kWayBasket) {
     // The basket's current volume: the top of the first track's state.
     DPath<D> c0;
     LoadState(cur, 0, c0);
-    if (ValidState(g, c0) && ValidState(g, c)) {
-      FindNextBoundaryAndStepBasket<D, M>(g, V3{a.x[i], a.y[i], a.z[i]}, V3{a.dx[i], a.dy[i], a.dz[i]}, c, o, ps,
-                                          step, c0.Top());
-    } else {
-      o = c;
-      if (c.level != 0) step = __builtin_nan("");
-    }
-  } else if (ValidState(g, c)) {
-    FindNextBoundaryAndStep<D, false, M, MX>(g, V3{a.x[i], a.y[i], a.z[i]}, V3{a.dx[i], a.dy[i], a.dz[i]}, c, o, ps,
-                                         step, a.kind);
-  } else {
+    valid = valid && ValidState(g, c0);
+    vol = c0.Top();
+  }
+  if (valid)
+    FindNextBoundaryAndStep<D, M, Way>(g, V3{a.x[i], a.y[i], a.z[i]}, V3{a.dx[i], a.dy[i], a.dz[i]}, o, ps, step, vol);
+  else if (o.level != 0)
     // A state outside the world has no volume to step in and stays outside
     // (step 0); a malformed state is left as it is, with step NaN.
-    o = c;
-    if (c.level != 0) step = __builtin_nan("");
-  }
+    step = __builtin_nan("");
   StoreState(nxt, i, o);
   a.step[i] = step;
 }
 
 template <int D, uint32_t M>
-__global__ __launch_bounds__(kNavBlock) void SafetyKernel(const NavDev g, const double *__restrict__ x,
-                                                          const double *__restrict__ y, const double *__restrict__ z,
-                                                          uint64_t n, const vg_nav_states s, double *__restrict__ out) {
-  const uint64_t i = (uint64_t)blockIdx.x * kNavBlock + threadIdx.x;
+__global__ __launch_bounds__(kNavBlock) __attribute__((amdgpu_waves_per_eu(StepWaves(M)))) void SafetyKernel(
+    const NavDev g, const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z, uint64_t n,
+    const vg_nav_states s, double *__restrict__ out, int shift) {
+  const uint64_t i = TrackOf((uint64_t)blockIdx.x * kNavBlock + threadIdx.x, shift, n);
   if (i >= n) return;
   DPath<D> c;
   LoadState(s, i, c);
@@ -154,65 +169,22 @@ struct TraceArgs {
   int32_t *exact;
   uint64_t n;
   double pstep;
-  int32_t kind;
   int32_t max_steps;
-  int32_t stage_lo, stage_hi;  // daughter slots copied to LDS first (none when equal)
-  int32_t stage_bounds;        // 1: their FP32 bound records too (mixed kernel)
-  int32_t pad;
+  int32_t shift;  // LanesShift(n)
 };
 
-// The world volume's daughter-slot boxes (8 floats each) are staged in LDS
-// by the trace kernel when they take at most this many bytes: 20 resident
-// workgroups per CU (five waves per SIMD, two waves a workgroup) then still
-// fit in 160 KiB.
-constexpr size_t kNavBoxLds = 8192;
-// ... and, in the mixed kernel, their FP32 bound records (144 bytes each)
-// when those take at most this many bytes more.
-constexpr size_t kNavBoundLds = 9216;
 
-// Occupancy floor of the fused trace kernel over the basic shape set: it is
-// latency-bound, and 5 waves per SIMD (instead of the 3 its 145 VGPRs allow,
-// at the price of spilled registers) measured 0.91 -> 1.01 G steps/s on the
-// nested geometry (4 waves: 1.00, 6: 0.89).  The per-step and serving
-// kernels measured no better with a floor.
-constexpr int TraceWaves(uint32_t m) { return m == kBasicShapes ? 5 : 1; }
-
-template <int D, uint32_t M, bool MX>
+template <int D, uint32_t M, int Way>
 __global__ __launch_bounds__(kNavBlock) __attribute__((amdgpu_waves_per_eu(TraceWaves(M)))) void TraceKernel(
     const NavDev g, const TraceArgs a) {
-  extern __shared__ __align__(16) float nav_boxes[];
-  NavDev gl = g;
-  if (a.stage_hi > a.stage_lo) {  // uniform over the grid
-    const int nf = 8 * (a.stage_hi - a.stage_lo);
-    const float *src = g.slot_box + 8 * (size_t)a.stage_lo;
-    for (int j = threadIdx.x; j < nf; j += kNavBlock) nav_boxes[j] = src[j];
-    __syncthreads();
-    gl.lds_box = nav_boxes;
-    gl.lds_lo = a.stage_lo;
-    gl.lds_hi = a.stage_hi;
-    if constexpr (MX) {
-      if (a.stage_bounds) {  // uniform over the grid
-        // Records follow the boxes (8 floats a slot keep them 16-byte aligned).
-        constexpr int kRec = (int)(sizeof(B32) / sizeof(uint32_t));
-        uint32_t *dst = reinterpret_cast<uint32_t *>(nav_boxes + nf);
-        const int nr = kRec * (a.stage_hi - a.stage_lo);
-        for (int j = threadIdx.x; j < nr; j += kNavBlock) {
-          const int slot = a.stage_lo + j / kRec;
-          dst[j] = reinterpret_cast<const uint32_t *>(g.b32 + g.daughters[slot])[j % kRec];
-        }
-        __syncthreads();
-        gl.lds_bound = reinterpret_cast<const B32 *>(dst);
-      }
-    }
-  }
-  const uint64_t i = (uint64_t)blockIdx.x * kNavBlock + threadIdx.x;
+  const uint64_t i = TrackOf((uint64_t)blockIdx.x * kNavBlock + threadIdx.x, a.shift, a.n);
   if (i >= a.n) return;
   V3 p{a.x[i], a.y[i], a.z[i]};
   const V3 d{a.dx[i], a.dy[i], a.dz[i]};
   double dist;
   uint64_t h;
   int nexact;
-  const int k = TraceOne<D, false, M, MX>(gl, p, d, a.pstep, a.kind, a.max_steps, dist, h, nexact);
+  const int k = TraceOne<D, M, Way>(g, p, d, a.pstep, a.max_steps, dist, h, nexact);
   a.nsteps[i] = k;
   a.fx[i] = p.x;
   a.fy[i] = p.y;
@@ -222,30 +194,21 @@ __global__ __launch_bounds__(kNavBlock) __attribute__((amdgpu_waves_per_eu(Trace
   if (a.exact) a.exact[i] = nexact;
 }
 
-NavDev Dev(const vg_geometry *g) {
-  NavDev d;
-  d.placed = g->d_placed;
-  d.params = g->d_params;
-  d.daughters = g->d_daughters;
-  d.aabb = g->d_aabb;
-  d.b32 = g->d_b32;
-  d.b32side = g->d_b32side;
-  d.slot_box = g->d_slot_aabb;
-  d.world = g->world;
-  d.n_placed = (int32_t)g->placed.size();
-  d.n_daughters = (int32_t)g->daughters.size();
-  d.pad = 0;
-  return d;
+unsigned Blocks(uint64_t n, int shift) {
+  const uint64_t per = (uint64_t)(kNavBlock / 64) << shift;
+  return (unsigned)((n + per - 1) / per);
 }
-
-unsigned Blocks(uint64_t n) { return (unsigned)((n + kNavBlock - 1) / kNavBlock); }
 
 }  // namespace
 
 int NavLocate(const vg_geometry *g, const double *x, const double *y, const double *z, uint64_t n,
               const vg_nav_states &s, hipStream_t st) {
   if (n == 0) return VG_OK;
-  VGA_NAV_VARIANTS(g, LocateKernel, dim3(Blocks(n)), dim3(kNavBlock), 0, st, Dev(g), x, y, z, n, s);
+  const int shift = LanesShift(n);
+  WithVariant(g, [&](auto D, auto M) {
+    hipLaunchKernelGGL((LocateKernel<D.value, M.value>), dim3(Blocks(n, shift)), dim3(kNavBlock), 0, st, DeviceNav(g),
+                       x, y, z, n, s, shift);
+  });
   return CheckHip(hipGetLastError(), "locate launch");
 }
 
@@ -253,16 +216,31 @@ int NavStep(const vg_geometry *g, int kind, const double *x, const double *y, co
             const double *dy, const double *dz, const double *pstep, uint64_t n, const vg_nav_states &cur,
             const vg_nav_states &nxt, double *step, hipStream_t st) {
   if (n == 0) return VG_OK;
-  StepArgs a{x, y, z, dx, dy, dz, pstep, step, n, kind, 0};
-  VGA_NAV_VARIANTS_MX(g, kind == VG_NAV_ABBOX_MIXED, StepKernel, dim3(Blocks(n)), dim3(kNavBlock), 0, st, Dev(g), a,
-                      cur, nxt);
+  const StepArgs a{x, y, z, dx, dy, dz, pstep, step, n, LanesShift(n), 0};
+  const dim3 blocks(Blocks(n, a.shift)), threads(kNavBlock);
+  if (kind == VG_NAV_SIMPLE)
+    WithVariant(g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+    });
+  else if (kind == VG_NAV_SIMPLE_BASKET)
+    WithVariant(g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayBasket>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+    });
+  else
+    WithVariant(g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+    });
   return CheckHip(hipGetLastError(), "step launch");
 }
 
 int NavSafety(const vg_geometry *g, const double *x, const double *y, const double *z, uint64_t n,
               const vg_nav_states &s, double *out, hipStream_t st) {
   if (n == 0) return VG_OK;
-  VGA_NAV_VARIANTS(g, SafetyKernel, dim3(Blocks(n)), dim3(kNavBlock), 0, st, Dev(g), x, y, z, n, s, out);
+  const int shift = LanesShift(n);
+  WithVariant(g, [&](auto D, auto M) {
+    hipLaunchKernelGGL((SafetyKernel<D.value, M.value>), dim3(Blocks(n, shift)), dim3(kNavBlock), 0, st, DeviceNav(g),
+                       x, y, z, n, s, out, shift);
+  });
   return CheckHip(hipGetLastError(), "safety launch");
 }
 
@@ -270,22 +248,16 @@ int NavTrace(const vg_geometry *g, int kind, const double *x, const double *y, c
              const double *dy, const double *dz, uint64_t n, double pstep, int max_steps, int32_t *nsteps, double *fx,
              double *fy, double *fz, double *travelled, uint64_t *hash, int32_t *exact, hipStream_t st) {
   if (n == 0) return VG_OK;
-  TraceArgs a{x, y, z, dx, dy, dz, nsteps, fx, fy, fz, travelled, hash, exact, n, pstep, kind, max_steps, 0, 0};
-  const PlacedRec *w = g->world >= 0 ? &g->placed[g->world] : nullptr;
-  const size_t box_bytes = w ? 8 * sizeof(float) * (size_t)(w->dend - w->dbegin) : 0;
-  size_t lds = 0;
-  if (box_bytes > 0 && box_bytes <= kNavBoxLds) {
-    a.stage_lo = w->dbegin;
-    a.stage_hi = w->dend;
-    lds = box_bytes;
-    const size_t bound_bytes = sizeof(B32) * (size_t)(w->dend - w->dbegin);
-    if (kind == VG_NAV_ABBOX_MIXED && g->d_b32 && bound_bytes <= kNavBoundLds) {
-      a.stage_bounds = 1;
-      lds += bound_bytes;
-    }
-  }
-  VGA_NAV_VARIANTS_MX(g, kind == VG_NAV_ABBOX_MIXED, TraceKernel, dim3(Blocks(n)), dim3(kNavBlock), lds, st, Dev(g),
-                      a);
+  const TraceArgs a{x, y, z, dx, dy, dz, nsteps, fx, fy, fz, travelled, hash, exact, n, pstep, max_steps, LanesShift(n)};
+  const dim3 blocks(Blocks(n, a.shift)), threads(kNavBlock);
+  if (kind == VG_NAV_SIMPLE)
+    WithVariant(g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g), a);
+    });
+  else
+    WithVariant(g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g), a);
+    });
   return CheckHip(hipGetLastError(), "trace launch");
 }
 

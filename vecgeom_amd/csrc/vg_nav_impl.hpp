@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <type_traits>
 #include <cstdint>
 #if defined(VGA_NAV_HOST_CHECKS)
 #include <cstdio>
@@ -22,7 +23,7 @@
 #else
 #define VGA_NAV_CHECK(cond, msg) ((void)0)
 #endif
-#define VGA_NAV inline __host__ __device__
+#define VGA_NAV __host__ __device__ __forceinline__
 
 #include "shapes.hpp"
 #include "vg_internal.hpp"
@@ -33,61 +34,54 @@ namespace nav {
 constexpr float kInfF = __builtin_huge_valf();
 
 struct NavDev {
-  const PlacedRec *placed;
-  const double *params;
-  const int32_t *daughters;
-  const float *aabb;
-  const B32 *b32;        // FP32 bound records (mixed-precision navigator)
-  const float *b32side;  // their variable-length data
-  const float *slot_box; // daughter boxes in slot order, 8 floats each
+  const NavRec *nav;            // per placed volume
+  const PlacedRec *placed;      // full placements (kNavMatrix)
+  const double *params;         // parameter blocks (kFormGeneral)
+  const float *slot_box;        // daughter boxes in slot order, 8 floats each
+  const DaughterIndex *dindex;  // daughter indexes (NavRec::index)
+  const uint64_t *dmasks;       // their masks
   int32_t world;
   int32_t n_placed;
   int32_t n_daughters;
-  int32_t pad;
-  // Slots [lds_lo, lds_hi) -- the world volume's daughters -- read from a
-  // copy in LDS made by the trace kernel (none elsewhere).
-  const float *lds_box = nullptr;
-  int32_t lds_lo = 0;
-  int32_t lds_hi = 0;
-  // The FP32 bound records of the same slots' daughters, in slot order
-  // (mixed trace kernel only; null elsewhere).
-  const B32 *lds_bound = nullptr;
-  VGA_NAV const PlacedRec &Pv(int id) const {
+  int32_t n_index;
+  int32_t n_masks;
+  VGA_NAV const NavRec &Nav(int id) const {
     VGA_NAV_CHECK(id >= 0 && id < n_placed, "placed id out of range");
-    return placed[id];
-  }
-  VGA_NAV int Daughter(int k) const {
-    VGA_NAV_CHECK(k >= 0 && k < n_daughters, "daughter slot out of range");
-    return daughters[k];
-  }
-  VGA_NAV const float *Box(int id) const {
-    VGA_NAV_CHECK(id >= 0 && id < n_placed, "box id out of range");
-    return aabb + 6 * (size_t)id;
+    return nav[id];
   }
   VGA_NAV const float *SlotBox(int k) const {
     VGA_NAV_CHECK(k >= 0 && k < n_daughters, "box slot out of range");
-    if (k >= lds_lo && k < lds_hi) return lds_box + 8 * (k - lds_lo);
     return slot_box + 8 * (size_t)k;
   }
-  VGA_NAV const B32 &Bound(int id) const {
-    VGA_NAV_CHECK(id >= 0 && id < n_placed, "bound id out of range");
-    return b32[id];
+  VGA_NAV int Daughter(int k) const {
+    int id;
+    __builtin_memcpy(&id, SlotBox(k) + 6, sizeof id);
+    return id;
   }
-  // The bound record of daughter slot k, whose placed id is id.
-  VGA_NAV const B32 &SlotBound(int k, int id) const {
-    if (lds_bound && k >= lds_lo && k < lds_hi) return lds_bound[k - lds_lo];
-    return Bound(id);
+  VGA_NAV const DaughterIndex &Index(int i) const {
+    VGA_NAV_CHECK(i >= 0 && i < n_index, "daughter index out of range");
+    return dindex[i];
+  }
+  VGA_NAV uint64_t Mask(int i) const {
+    VGA_NAV_CHECK(i >= 0 && i < n_masks, "daughter mask out of range");
+    return dmasks[i];
   }
 };
 
-// Shape sets of specialised navigators (bit t: shape type t).
-constexpr uint32_t kAllShapes = (1u << VG_BOX) | (1u << VG_TUBE) | (1u << VG_ORB) | (1u << VG_SPHERE) |
+// Shape sets of specialised navigators (bit t: shape type t; bit 0: a Tube
+// with a phi section).
+constexpr uint32_t kPhiTube = 1u;
+constexpr uint32_t kAllShapes = kPhiTube | (1u << VG_BOX) | (1u << VG_TUBE) | (1u << VG_ORB) | (1u << VG_SPHERE) |
                                 (1u << VG_CONE) | (1u << VG_TRD) | (1u << VG_TRAPEZOID) |
                                 (1u << VG_PARALLELEPIPED) | (1u << VG_PARABOLOID) | (1u << VG_TORUS) |
                                 (1u << VG_POLYCONE) | (1u << VG_POLYHEDRON);
-// Box, Tube, Orb and Trd: the fused trace kernel needs 145 VGPRs with these
-// alone (three waves per SIMD) against 230 with every shape (two).
+// Box, Tube, Orb and Trd: evaluated from the volume's NavRec alone (but for
+// the phi tubes).
 constexpr uint32_t kBasicShapes = (1u << VG_BOX) | (1u << VG_TUBE) | (1u << VG_ORB) | (1u << VG_TRD);
+// The shapes of set M that are evaluated from their parameter blocks.
+constexpr uint32_t BlockShapes(uint32_t m) {
+  return (m & ~kBasicShapes & ~kPhiTube) | ((m & kPhiTube) ? (1u << VG_TUBE) : 0u);
+}
 
 // ------------------------------------------------------------ shape switch
 // Shape switch over the compile-time shape set M (bit t set: shape type t
@@ -205,6 +199,110 @@ VGA_NAV double DSafeOut(int type, const double *blk, V3 p) {
 #undef VGA_P
 #undef VGA_SHAPE_CASES
 
+// The first half of a NavRec, in registers.
+struct Head {
+  int code, index, dbegin, nd;
+  double s[6];
+};
+VGA_NAV Head LoadHead(const NavDev &g, int id) {
+  const NavRec &r = g.Nav(id);
+  Head h{r.code, r.index, r.dbegin, r.nd, {}};
+#pragma unroll
+  for (int i = 0; i < 6; ++i) h.s[i] = r.s[i];
+  return h;
+}
+
+// Calls f(shape, parameters) for the simple shapes, their parameter blocks
+// rebuilt from the record (the same operations as the host's constructors,
+// so the same bits; the unused members stay undefined), or general(type,
+// block) for the others.
+template <uint32_t M, bool Safety, class F, class G>
+VGA_NAV auto WithShape(const NavDev &g, int id, const Head &h, F f, G general) {
+  switch (h.code & kNavFormMask) {
+    case kFormBox:
+      if constexpr ((M >> VG_BOX) & 1u) return f(BoxS{}, BoxP{{h.s[0], h.s[1], h.s[2]}});
+      break;
+    case kFormTube:
+      if constexpr ((M >> VG_TUBE) & 1u) {
+        TubeP t;
+        t.rmin = h.s[0];
+        t.rmax = h.s[1];
+        t.z = h.s[2];
+        t.rmin2 = t.rmin * t.rmin;
+        t.rmax2 = t.rmax * t.rmax;
+        const double lo = t.rmin + kTolerance, hi = t.rmax - kTolerance;
+        t.tolIrmin2 = lo * lo;
+        t.tolIrmax2 = hi * hi;
+        t.hasRmin = t.rmin > 0 ? 1. : 0.;
+        t.hasPhi = 0.;
+        return f(TubeS{}, t);
+      }
+      break;
+    case kFormTrd:
+      if constexpr ((M >> VG_TRD) & 1u) {
+        TrdP t;
+        t.dx1 = h.s[0];
+        t.dx2 = h.s[1];
+        t.dy1 = h.s[2];
+        t.dy2 = h.s[3];
+        t.dz = h.s[4];
+        t.x2minusx1 = t.dx2 - t.dx1;
+        t.y2minusy1 = t.dy2 - t.dy1;
+        t.halfx1plusx2 = 0.5 * (t.dx1 + t.dx2);
+        t.halfy1plusy2 = 0.5 * (t.dy1 + t.dy2);
+        t.dztimes2 = t.dz * 2;
+        t.fx = h.s[5];
+        t.fy = 0.5 * (t.dy1 - t.dy2) / t.dz;
+        if constexpr (Safety) {
+          t.calfx = 1. / Sqrt(1.0 + t.fx * t.fx);
+          t.calfy = 1. / Sqrt(1.0 + t.fy * t.fy);
+        }
+        t.varyingY = t.dy1 != t.dy2 ? 1. : 0.;
+        return f(TrdS{}, t);
+      }
+      break;
+    case kFormOrb:
+      if constexpr ((M >> VG_ORB) & 1u) return f(OrbS{}, OrbP{h.s[0], h.s[1], h.s[2], 0.});
+      break;
+  }
+  if constexpr (BlockShapes(M) != 0) {
+    const NavRec &r = g.Nav(id);
+    return general(r.type, g.params + r.param_off);
+  } else {
+    return decltype(f(BoxS{}, BoxP{}))(0);  // no such volume
+  }
+}
+template <uint32_t M>
+VGA_NAV bool NContains(const NavDev &g, int id, const Head &h, V3 p) {
+  return WithShape<M, false>(
+      g, id, h, [&](auto s, const auto &q) { return decltype(s)::Contains(q, p); },
+      [&](int type, const double *blk) { return DContains<BlockShapes(M)>(type, blk, p); });
+}
+template <uint32_t M>
+VGA_NAV double NDistIn(const NavDev &g, int id, const Head &h, V3 p, V3 d, double sm) {
+  return WithShape<M, false>(
+      g, id, h, [&](auto s, const auto &q) { return decltype(s)::DistanceToIn(q, p, d, sm); },
+      [&](int type, const double *blk) { return DDistIn<BlockShapes(M)>(type, blk, p, d, sm); });
+}
+template <uint32_t M>
+VGA_NAV double NDistOut(const NavDev &g, int id, const Head &h, V3 p, V3 d, double sm) {
+  return WithShape<M, false>(
+      g, id, h, [&](auto s, const auto &q) { return decltype(s)::DistanceToOut(q, p, d, sm); },
+      [&](int type, const double *blk) { return DDistOut<BlockShapes(M)>(type, blk, p, d, sm); });
+}
+template <uint32_t M>
+VGA_NAV double NSafeIn(const NavDev &g, int id, const Head &h, V3 p) {
+  return WithShape<M, true>(
+      g, id, h, [&](auto s, const auto &q) { return decltype(s)::SafetyToIn(q, p); },
+      [&](int type, const double *blk) { return DSafeIn<BlockShapes(M)>(type, blk, p); });
+}
+template <uint32_t M>
+VGA_NAV double NSafeOut(const NavDev &g, int id, const Head &h, V3 p) {
+  return WithShape<M, true>(
+      g, id, h, [&](auto s, const auto &q) { return decltype(s)::SafetyToOut(q, p); },
+      [&](int type, const double *blk) { return DSafeOut<BlockShapes(M)>(type, blk, p); });
+}
+
 // ------------------------------------------------------------------ path
 template <int D>
 struct DPath {
@@ -281,12 +379,31 @@ VGA_NAV void MultiplyFromRight(Xf &m, const Xf &rhs, int kind) {
   }
 }
 
-VGA_NAV void LoadXf(const PlacedRec &r, Xf &x) {
+// The placement of volume id with code `code`: only the parts that are not
+// the identity's are read.
+VGA_NAV Xf LoadXf(const NavDev &g, int id, int code) {
+  Xf x{{0., 0., 0.}, {1., 0., 0., 0., 1., 0., 0., 0., 1.}};
+  if (code & (kNavMoves | kNavTurns)) {
+    const NavRec &r = g.Nav(id);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) x.t[i] = r.xf.t[i];
+    for (int i = 0; i < 3; ++i) x.t[i] = r.t[i];
+    if (code & kNavTurns) {
+      x.r[0] = r.r[0];
+      x.r[1] = r.r[1];
+      x.r[3] = r.r[2];
+      x.r[4] = r.r[3];
+    }
+  } else if (code & kNavMatrix) {
+    VGA_NAV_CHECK(id >= 0 && id < g.n_placed, "placed id out of range");
+    const Xf &m = g.placed[id].xf;
 #pragma unroll
-  for (int i = 0; i < 9; ++i) x.r[i] = r.xf.r[i];
+    for (int i = 0; i < 3; ++i) x.t[i] = m.t[i];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) x.r[i] = m.r[i];
+  }
+  return x;
 }
+VGA_NAV int KindOf(int code) { return (code >> kNavKindShift) & 3; }
 
 // The unspecialised Transform (all terms), used on TopMatrix and on the
 // pushed point after a boundary.
@@ -315,122 +432,210 @@ VGA_NAV Xf TopMatrix(const NavDev &g, const DPath<D> &s) {
 #pragma unroll
   for (int i = 0; i < 9; ++i) m.r[i] = (i % 4 == 0) ? 1. : 0.;
   for (int l = 1; l < s.level; ++l) {
-    const PlacedRec &r = g.Pv(s.Get(l));
-    Xf x;
-    LoadXf(r, x);
-    MultiplyFromRight(m, x, r.xfkind);
+    const int id = s.Get(l), code = g.Nav(id).code;
+    if (KindOf(code) != kXfIdentity) MultiplyFromRight(m, LoadXf(g, id, code), KindOf(code));
   }
   return m;
 }
 
-// Contains of a placed volume on a point of its mother frame; the local
-// point is returned through `local` (meaningful when the result is true).
-// Mixed: the FP32 filter decides first (vg_bound32.hpp: a point farther
-// from the surface than the bound's rounding margin is classified exactly
-// as the FP64 Contains classifies it), and the FP64 Contains runs only for
-// points it leaves undecided.
-template <uint32_t M = kAllShapes>
-VGA_NAV bool PlacedContains(const NavDev &g, int pv, V3 p, V3 &local, bool mixed = false) {
-  int c = -1;
-  if (mixed) {
-    c = Classify32<M>(g.Bound(pv), g.b32side, F3{(float)p.x, (float)p.y, (float)p.z});
-    if (c == kOutside) return false;
-  }
-  const PlacedRec &r = g.Pv(pv);
-  Xf x;
-  LoadXf(r, x);
-  local = XfPointRt(x, r.xfkind, p);
-  return c == kInside || DContains<M>(r.type, g.params + r.param_off, local);
-}
+// ---------------------------------------------------- daughters on the way
+// The daughters of a volume that can meet a stretch of a ray (or hold a
+// point), as bit masks over its daughter slots (vg_daughter_index.hpp): word
+// w of a mask is slots dbegin + 64 w + bit.
+struct Meet {
+  int nd, words, axes;         // axes: NavRec::code
+  const DaughterIndex *index;  // null: every daughter
+  int l0, l1, l2, h0, h1, h2;  // rows of the stretch's ends in the tables
 
-template <uint32_t M = kAllShapes>
-VGA_NAV double PlacedDistIn(const NavDev &g, int pv, V3 p, V3 d, double sm) {
-  const PlacedRec &r = g.Pv(pv);
-  Xf x;
-  LoadXf(r, x);
-  return DDistIn<M>(r.type, g.params + r.param_off, XfPointRt(x, r.xfkind, p), XfDirRt(x, r.xfkind, d), sm);
+  VGA_NAV Meet(const NavDev &g, int code, int ix, int n, bool use) {
+    nd = n;
+    words = (nd + 63) >> 6;
+    axes = code >> kNavAxesShift;
+    index = use && ix >= 0 ? &g.Index(ix) : nullptr;
+    l0 = l1 = l2 = h0 = h1 = h2 = 0;
+  }
+  VGA_NAV int Count() const { return axes & 3; }
+  VGA_NAV int Row(const DaughterAxis &ax, float u) const {
+    const float s = (u - ax.lo) * ax.inv;
+    const int i = s < (float)(ax.slices - 1) ? (s > 0.f ? (int)s : 0) : ax.slices - 1;
+    return ax.off + i * (2 * words);
+  }
+  template <int A, class F>
+  VGA_NAV void Axis(F f, int &l, int &h) {
+    if (A >= Count()) return;
+    float u0, u1;
+    f((axes >> (kNavCoordShift - kNavAxesShift + 2 * A)) & 3, u0, u1);
+    const DaughterAxis ax = index->axis[A];
+    l = Row(ax, u0);
+    h = Row(ax, u1);
+  }
+  template <class F>
+  VGA_NAV void Axes(F f) {
+    if (!index) return;
+    Axis<0>(f, l0, h0);
+    Axis<1>(f, l1, h1);
+    Axis<2>(f, l2, h2);
+  }
+  // The points within `reach` of p in every coordinate.
+  VGA_NAV void Around(F3 p, float reach) {
+    const float e = reach + 2e-6f * (Abs1(p) + reach);
+    Axes([&](int c, float &u0, float &u1) {
+      const float u = c == 0 ? p.x : c == 1 ? p.y : c == 2 ? p.z : __builtin_sqrtf(p.x * p.x + p.y * p.y);
+      u0 = u - e;
+      u1 = u + e;
+    });
+  }
+  // The stretch p + t d, t0 <= t <= t1; its coordinates are widened by the
+  // rounding of their float evaluation.
+  VGA_NAV void Stretch(F3 p, F3 d, float t0, float t1) {
+    const float e = 2e-6f * (Abs1(p) + t1);
+    const F3 a{p.x + t0 * d.x, p.y + t0 * d.y, p.z + t0 * d.z}, b{p.x + t1 * d.x, p.y + t1 * d.y, p.z + t1 * d.z};
+    Axes([&](int c, float &u0, float &u1) {
+      if (c < 3) {
+        const float q = c == 0 ? a.x : c == 1 ? a.y : a.z, r = c == 0 ? b.x : c == 1 ? b.y : b.z;
+        u0 = q < r ? q : r;
+        u1 = q < r ? r : q;
+      } else {
+        // rho^2 is convex along the ray: largest at an end, smallest at the
+        // closest approach to the axis.
+        const float aa = d.x * d.x + d.y * d.y;
+        float tm = aa > 0.f ? -(p.x * d.x + p.y * d.y) / aa : t0;
+        tm = tm > t0 ? (tm < t1 ? tm : t1) : t0;
+        const float xm = p.x + tm * d.x, ym = p.y + tm * d.y;
+        const float ra = a.x * a.x + a.y * a.y, rb = b.x * b.x + b.y * b.y;
+        u0 = __builtin_sqrtf(xm * xm + ym * ym);
+        u1 = __builtin_sqrtf(ra < rb ? rb : ra);
+      }
+      u0 -= e;
+      u1 += e;
+    });
+  }
+  static VGA_NAV float Abs1(F3 p) { return __builtin_fabsf(p.x) + __builtin_fabsf(p.y) + __builtin_fabsf(p.z); }
+  VGA_NAV uint64_t Full(int w) const { return nd - 64 * w >= 64 ? ~0ull : (1ull << (nd - 64 * w)) - 1; }
+  VGA_NAV uint64_t Mask(const NavDev &g, int w) const {
+    uint64_t m = Full(w);
+    if (!index) return m;
+    const int c = Count();
+    if (c > 0) m &= g.Mask(l0 + w) & g.Mask(h0 + words + w);
+    if (c > 1) m &= g.Mask(l1 + w) & g.Mask(h1 + words + w);
+    if (c > 2) m &= g.Mask(l2 + w) & g.Mask(h2 + words + w);
+    return m;
+  }
+};
+// The part of a ray's way t >= 0 that lies in the box of all the index's
+// daughters, widened by the rounding of t; false when there is none.
+VGA_NAV bool Clip(const DaughterIndex &ix, F3 p, F3 d, float &t0, float &t1) {
+  t0 = 0.f;
+  t1 = kInfF;
+  const float pv[3] = {p.x, p.y, p.z}, dv[3] = {d.x, d.y, d.z};
+  const float e = 4e-6f * Meet::Abs1(p);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float a = ix.lo[c] - e - pv[c], b = ix.hi[c] + e - pv[c];
+    if (__builtin_fabsf(dv[c]) > 1e-12f) {
+      const float inv = 1.f / dv[c], u = a * inv, v = b * inv;
+      t0 = t0 > (u < v ? u : v) ? t0 : (u < v ? u : v);
+      t1 = t1 < (u < v ? v : u) ? t1 : (u < v ? v : u);
+    } else if (a > 1e-3f || b < -1e-3f) {
+      // Moves less than 1e-3 in this coordinate over 1e9.
+      return false;
+    }
+  }
+  t0 = t0 * (1.f - 4e-6f);
+  t1 = t1 * (1.f + 4e-6f);
+  return t0 <= t1;
 }
+// A point whose coordinates the index's floats hold.
+VGA_NAV bool Finite(V3 p) { return p.Mag2() < 1e30; }
 
 // ----------------------------------------------------------- locate family
-template <int D, uint32_t M = kAllShapes>
-VGA_NAV int LocatePoint(const NavDev &g, int vol, V3 point, DPath<D> &path, bool top, bool mixed = false) {
-  int cand = vol;
-  V3 tmp = point;
-  if (top) {
-    const PlacedRec &r = g.Pv(vol);
-    cand = DContains<M>(r.type, g.params + r.param_off, point) ? vol : -1;
-  }
-  if (cand >= 0) {
-    path.Push(cand);
-    bool deeper = true;
-    while (deeper) {
-      const int db = g.Pv(cand).dbegin, de = g.Pv(cand).dend;
-      if (de <= db) break;
-      deeper = false;
-      for (int k = db; k < de; ++k) {
-        const int nx = g.Daughter(k);
-        V3 tp;
-        if (PlacedContains<M>(g, nx, tmp, tp, mixed)) {
+// The daughter scan below tests only the daughters near the point, in the
+// order of the full scan: a daughter that is not near cannot contain it.
+
+// Where a track goes on: from volume vol, already on its path, at `point` of
+// vol's frame.  vol < 0: nowhere.
+struct Target {
+  int vol, excluded;
+  V3 point;
+  bool down;
+};
+
+// Descends from the target: the first daughter in the scan's order that
+// contains the point, and so on down; returns the deepest volume.  Rising
+// daughter index (SimpleNavigator::LocatePoint) or, with `down`, falling and
+// never into `excluded` (LocatePointExclVolume).
+template <int D, uint32_t M>
+VGA_NAV int Descend(const NavDev &g, Target t, DPath<D> &path) {
+  bool deeper = t.vol >= 0;
+  while (deeper) {
+    const NavRec &C = g.Nav(t.vol);
+    const int db = C.dbegin, nd = C.nd;
+    if (nd <= 0) break;
+    deeper = false;
+    Meet near(g, C.code, C.index, nd, Finite(t.point));
+    near.Around(F3{(float)t.point.x, (float)t.point.y, (float)t.point.z}, 0.f);
+    for (int j = 0; j < near.words && !deeper; ++j) {
+      const int w = t.down ? near.words - 1 - j : j;
+      uint64_t m = near.Mask(g, w);
+      while (m && !deeper) {
+        const int bit = t.down ? 63 - __builtin_clzll(m) : __builtin_ctzll(m);
+        m ^= 1ull << bit;
+        const int nx = g.Daughter(db + 64 * w + bit);
+        if (t.down && nx == t.excluded) continue;
+        const Head h = LoadHead(g, nx);
+        const V3 local = XfPointRt(LoadXf(g, nx, h.code), KindOf(h.code), t.point);
+        if (NContains<M>(g, nx, h, local)) {
           path.Push(nx);
-          tmp = tp;
-          cand = nx;
+          t.point = local;
+          t.vol = nx;
           deeper = true;
-          break;
         }
       }
     }
   }
-  return cand;
+  return t.vol;
 }
 
-template <int D, uint32_t M = kAllShapes>
-VGA_NAV int LocatePointExcl(const NavDev &g, int vol, int excluded, V3 point, DPath<D> &path, bool mixed = false) {
-  int cand = vol;
-  V3 tmp = point;
-  path.Push(cand);
-  bool deeper = true;
-  while (deeper) {
-    const int db = g.Pv(cand).dbegin, de = g.Pv(cand).dend;
-    if (de <= db) break;
-    deeper = false;
-    for (int k = de - 1; k >= db; --k) {
-      const int nx = g.Daughter(k);
-      V3 tp;
-      if (nx != excluded && PlacedContains<M>(g, nx, tmp, tp, mixed)) {
-        path.Push(nx);
-        tmp = tp;
-        cand = nx;
-        deeper = true;
-        break;
-      }
-    }
-  }
-  return cand;
+// SimpleNavigator::LocatePoint from the world.
+template <int D, uint32_t M>
+VGA_NAV Target FromWorld(const NavDev &g, V3 point, DPath<D> &path) {
+  if (!NContains<M>(g, g.world, LoadHead(g, g.world), point)) return Target{-1, -1, point, false};
+  path.Push(g.world);
+  return Target{g.world, -1, point, false};
 }
 
-template <int D, uint32_t M = kAllShapes>
-VGA_NAV int Relocate(const NavDev &g, V3 localpoint, DPath<D> &path, bool mixed = false) {
+// LocatePoint in daughter nv, entered at `point` of its mother's frame.
+template <int D>
+VGA_NAV Target Into(const NavDev &g, int nv, V3 point, DPath<D> &path) {
+  path.Push(nv);
+  return Target{nv, -1, ApplyGeneric(LoadXf(g, nv, g.Nav(nv).code), point), false};
+}
+
+// RelocatePointFromPath: up to the first volume of the path that contains
+// the point.
+template <int D, uint32_t M>
+VGA_NAV Target Relocate(const NavDev &g, V3 point, DPath<D> &path) {
   int mother = path.Top();
-  if (mother >= 0) {
-    V3 tmp = localpoint;
-    while (mother >= 0) {
-      const PlacedRec &r = g.Pv(mother);
-      if (DContains<M>(r.type, g.params + r.param_off, tmp)) break;
-      path.Pop();
-      Xf x;
-      LoadXf(r, x);
-      tmp = InversePoint(x, tmp);
-      mother = path.Top();
-    }
-    if (mother >= 0) {
-      path.Pop();
-      return LocatePointExcl<D, M>(g, mother, mother, tmp, path, mixed);
-    }
+  while (mother >= 0) {
+    const Head h = LoadHead(g, mother);
+    if (NContains<M>(g, mother, h, point)) break;
+    path.Pop();
+    point = InversePoint(LoadXf(g, mother, h.code), point);
+    mother = path.Top();
   }
-  return mother;
+  return Target{mother, mother, point, true};
 }
+
+// The navigators, as template arguments: each kernel carries the code of one
+// (the mixed ABBox navigator is the ABBox one: its daughters are preselected
+// in FP32 by the daughter index, and its results are the same).
+enum NavWay : int { kWayAbbox, kWaySimple, kWayBasket, kWayAbboxSorted };
+VGA_NAV constexpr bool Abbox(int way) { return way == kWayAbbox || way == kWayAbboxSorted; }
 
 // ------------------------------------------------------------ ABBox search
+constexpr float kReach = 4.f;  // growth of the searched stretch
+constexpr float kNear = 8.f;   // a step within this many first stretches is searched at once
+
 struct Ray {
   float p[3];
   float inv[3];
@@ -480,190 +685,162 @@ VGA_NAV Ray MakeRay(V3 lp, V3 ld) {
 // the exact sorted-order walk was needed.  ExactOnly skips the order-free
 // walk (used by the host-side checks of the exact walk).
 //
-// Mixed (VG_NAV_ABBOX_MIXED): before its FP64 Contains and DistanceToIn, a
-// hit daughter is skipped when its FP32 lower bound on the distance from the
-// point (vg_bound32.hpp) exceeds the best step found so far by more than
-// the bound's rounding margin and 1e-6 mm.  Such a daughter cannot contain
-// the point, and its DistanceToIn (the ray's distance to its surface, never
-// shorter than the Euclidean distance by more than the tolerance) exceeds
-// the final step, so it can neither win nor tie: the walk's result is
-// unchanged.
+// The walk searches the ray in growing stretches from its start: the
+// daughters whose extents the stretch can meet, less those seen already, in
+// index order; it ends with the first stretch that reaches the best step
+// found.  Every daughter left lies beyond that step: it cannot contain the
+// start, and its DistanceToIn exceeds the step, so it can neither win nor
+// tie.  The order does not matter to the outcome.  That argument needs the
+// shapes' distances to be distances, which takes a unit direction; any other
+// direction takes every daughter at once.
 //
-// In the mixed form the walk runs in two phases per group of up to 64
-// daughters: the box tests alone (a short loop whose loads do not depend on
-// each other), recording hits in a bit mask, then the hit daughters in index
-// order -- the order of the single loop of the FP64 form, which measured
-// faster there.
-template <bool ExactOnly = false, uint32_t M = kAllShapes, bool Mixed = false>
-VGA_NAV int AbboxCandidates(const NavDev &g, int db, int de, V3 lp, V3 ld, double &step, int &next) {
+// Where the outcome does depend on the order the walk starts again and takes
+// the hits in ascending (entry distance, daughter index) order, the order of
+// a stable sort of the hit list, by repeated selection of the next one.  Both
+// orders share the code that evaluates a daughter.
+// Where the next stretch to search ends, given its begin T0, the end T of
+// the one searched before (0: none) and the step known: at the step where
+// that is near, else kReach times as far as before, and never beyond T1.
+VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
+  if (!way.index) return 0.f;
+  const float first = way.index->first;
+  const float far = T > 0.f ? T0 + kReach * (T - T0) : T0 + first;
+  const double to = step * (1. + 1e-6) + 1e-6;  // not below step as a float
+  const float end = to <= (double)(T0 + kNear * first) || to <= (double)far ? (float)to : far;
+  return end < T1 ? end : T1;
+}
+
+// SimpleNavigator's loop over the daughters (kWaySimple, kWayBasket) is the
+// same search without the box tests: it takes the smallest DistanceToIn, of
+// equal ones the daughter with the lowest index (an index-order loop with a
+// strict comparison).
+template <uint32_t M, int Way>
+VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &step, int &next) {
+  const int db = C.dbegin;
   const Ray ray = MakeRay(lp, ld);
   const double step0 = step;
-  double best = step0;
-  int bk = -1, ties = 0;
-  bool exact = ExactOnly;
-  const F3 lp32{(float)lp.x, (float)lp.y, (float)lp.z};
-  // One hit daughter (slot k, box entry b); false ends the walk (exact path).
-  auto visit = [&](int k, float b) -> bool {
-    const int cand = g.Daughter(k);
-    if (Mixed) {
-      float so, si, m;
-      Bound32<M>(g.SlotBound(k, cand), g.b32side, lp32, so, si, m);
-      if ((double)so - (double)m > Max(best, 0.) + 1e-6) return true;
-    }
-    const PlacedRec &r = g.Pv(cand);
-    Xf x;
-    LoadXf(r, x);
-    const V3 tp = XfPointRt(x, r.xfkind, lp);
-    const double *blk = g.params + r.param_off;
-    if (b < 0.f && DContains<M>(r.type, blk, tp)) return false;
-    const double dd = DDistIn<M>(r.type, blk, tp, XfDirRt(x, r.xfkind, ld), step0);
-    if (dd < 0. || dd < (double)b) return false;
-    if (dd < best) {
-      best = dd;
-      bk = k - db;
-      ties = 1;
-    } else if (dd == best) {
-      ++ties;
-    }
-    return true;
-  };
-  if constexpr (!ExactOnly && Mixed) {
-    for (int base = db; base < de && !exact; base += 64) {
-      const int cnt = de - base < 64 ? de - base : 64;
-      uint64_t hits = 0;
-      for (int j = 0; j < cnt; ++j) hits |= (uint64_t)(IntersectBox(g.SlotBox(base + j), ray) < kInfF) << j;
-      while (hits && !exact) {
-        const int k = base + __builtin_ctzll(hits);
-        hits &= hits - 1;
-        exact = !visit(k, IntersectBox(g.SlotBox(k), ray));
-      }
-    }
-  } else if constexpr (!ExactOnly) {
-    for (int k = db; k < de && !exact; ++k) {
-      const float b = IntersectBox(g.SlotBox(k), ray);
-      if (b < kInfF) exact = !visit(k, b);
-    }
+  Meet way(g, C.code, C.index, C.nd, Finite(lp) && Abs(ld.Mag2() - 1.) < 1e-12);
+  const F3 fp{ray.p[0], ray.p[1], ray.p[2]}, fd{(float)ld.x, (float)ld.y, (float)ld.z};
+  // The stretch [T0, T] of the ray is searched next; beyond T1 it meets no
+  // daughter.
+  float T0 = 0.f, T1 = kInfF, T = 0.f;
+  int w = 0;
+  uint64_t m, seen = 0;
+  if (way.index && (!Clip(*way.index, fp, fd, T0, T1) || (double)T0 > step)) {
+    m = 0;
+    T = T1 = 0.f;
+    w = way.words;
+  } else {
+    T = Reach(way, T0, T1, 0.f, step);
+    way.Stretch(fp, fd, T0, T);
+    seen = m = way.Mask(g, 0);
   }
-  if (!exact && ties <= 1) {
-    step = best;
-    next = bk;
-    return 0;
-  }
-  // Exact walk: hits in ascending (entry distance, daughter index) order,
-  // the order of a stable sort of the hit list.
-  step = step0;
-  next = -1;
+  float behind = 0.f;
+  bool sorted = Way == kWayAbboxSorted;
+  int ties = 0;
   float lastb = -kInfF;
   int lastk = -1;
+  next = -1;
   while (true) {
-    float bb = kInfF;
-    int kk = -1;
-    for (int k = db; k < de; ++k) {
-      const float b = IntersectBox(g.SlotBox(k), ray);
-      if (!(b < kInfF)) continue;
-      const int kl = k - db;
-      const bool after = (b > lastb) || (b == lastb && kl > lastk);
-      if (after && (kk < 0 || b < bb)) {
-        bb = b;
-        kk = kl;
+    int k;
+    float b;
+    if (!sorted) {
+      if (!m) {
+        if (++w < way.words) {
+          m = way.Mask(g, w);
+          if (behind > 0.f) {
+            Meet before = way;
+            before.Stretch(fp, fd, T0, behind);
+            m &= ~before.Mask(g, w);
+          }
+        } else {
+          if (!way.index || T >= T1 || step <= (double)T) {
+            if (!Abbox(Way) || ties <= 1) return 0;
+            sorted = true;
+            step = step0;
+            next = -1;
+            continue;
+          }
+          behind = T;
+          T = Reach(way, T0, T1, T, step);
+          way.Stretch(fp, fd, T0, T);
+          w = 0;
+          const uint64_t all = way.Mask(g, 0);
+          m = all & ~seen;
+          seen = all;
+        }
+        continue;
       }
-    }
-    if (kk < 0) break;
-    lastb = bb;
-    lastk = kk;
-    const double hd = (double)bb;
-    if (step < hd) break;
-    const int cand = g.Daughter(db + kk);
-    if (hd < 0) {
-      V3 tp;
-      if (PlacedContains<M>(g, cand, lp, tp)) {
-        step = 0;
-        next = kk;
-        break;
+      k = 64 * w + __builtin_ctzll(m);
+      m &= m - 1;
+      if constexpr (Abbox(Way)) {
+        b = IntersectBox(g.SlotBox(db + k), ray);
+        if (!(b < kInfF)) continue;
+      } else {
+        b = 0.f;
       }
+    } else {
+      k = -1;
+      b = kInfF;
+      for (int j = 0; j < C.nd; ++j) {
+        const float bj = IntersectBox(g.SlotBox(db + j), ray);
+        const bool after = bj < kInfF && (bj > lastb || (bj == lastb && j > lastk));
+        if (after && (k < 0 || bj < b)) {
+          b = bj;
+          k = j;
+        }
+      }
+      if (k < 0 || step < (double)b) return 1;
+      lastb = b;
+      lastk = k;
     }
-    const double dd = PlacedDistIn<M>(g, cand, lp, ld, step);
-    if (dd < step) {
-      next = kk;
+    const int cand = g.Daughter(db + k);
+    const Head h = LoadHead(g, cand);
+    const Xf x = LoadXf(g, cand, h.code);
+    const V3 tp = XfPointRt(x, KindOf(h.code), lp);
+    const bool within = b < 0.f && NContains<M>(g, cand, h, tp);
+    if (within && sorted) {
+      step = 0;
+      next = k;
+      return 1;
+    }
+    // SimpleNavigator's step limit is the running step; with the index, whose
+    // order is another, the first one (no answer below the step depends on
+    // it for a unit direction).
+    const double sm = (Abbox(Way) ? sorted : !way.index) ? step : step0;
+    const double dd = NDistIn<M>(g, cand, h, tp, XfDirRt(x, KindOf(h.code), ld), sm);
+    if (!Abbox(Way)) {
+      if ((dd < step || (dd == step && k < next)) && !(Way == kWaySimple && __builtin_isinf(dd))) {
+        step = dd;
+        next = k;
+      }
+    } else if (sorted) {
+      if (dd < step) {
+        next = k;
+        step = dd;
+      }
+    } else if (within || dd < 0. || dd < (double)b) {
+      sorted = true;
+      step = step0;
+      next = -1;
+    } else if (dd < step) {
       step = dd;
+      next = k;
+      ties = 1;
+    } else if (dd == step) {
+      ++ties;
     }
   }
-  return 1;
 }
 
-// FindNextBoundaryAndStep of both navigators (kind 0 ABBox, 1 Simple).
-// Returns 1 if the ABBox walk took the exact path.
-// Mixed: the navigator of VG_NAV_ABBOX_MIXED (kind must then be that
-// navigator): FP32 filters in the daughter walk and in the locate scans.
-template <int D, bool ExactOnly = false, uint32_t M = kAllShapes, bool Mixed = false>
-VGA_NAV int FindNextBoundaryAndStep(const NavDev &g, V3 gp, V3 gd, const DPath<D> &cur, DPath<D> &nst,
-                                       double pstep, double &step, int kind) {
-  const Xf m = TopMatrix(g, cur);
-  const V3 lp = ApplyGeneric(m, gp);
-  const V3 ld = Rotate(m, gd);
-  const int cv = cur.Top();
-  const PlacedRec &C = g.Pv(cv);
-  const int db = C.dbegin, de = C.dend;
-  int next = -1;
-  int exact = 0;
-  step = DDistOut<M>(C.type, g.params + C.param_off, lp, ld, pstep);
-  nst = cur;
-  constexpr bool mixed = Mixed;
-  const bool abbox = kind == VG_NAV_ABBOX || kind == VG_NAV_ABBOX_MIXED;
-  if (abbox) {
-    if (step < 0.) step = kInfinity;
-    if (de > db) exact = AbboxCandidates<ExactOnly, M, Mixed>(g, db, de, lp, ld, step, next);
-    if (step > pstep) {
-      step = pstep;
-      nst.boundary = 0;
-      return exact;
-    }
-    nst.boundary = 1;
-    if (step > 1E30) {
-      step = 0;
-      nst.Pop();
-      return exact;
-    }
-    if (step < 0.) step = 0.;
-  } else {
-    if (step <= 0.) step = kInfinity;
-    for (int k = db; k < de; ++k) {
-      const double dd = PlacedDistIn<M>(g, g.Daughter(k), lp, ld, step);
-      const bool valid = dd < step && !__builtin_isinf(dd);
-      next = valid ? k - db : next;
-      step = valid ? dd : step;
-    }
-    if (step == kInfinity && pstep > 0.) {
-      step = 0;
-      nst.Pop();
-      nst.boundary = 1;
-      return 0;
-    }
-    if (step > pstep) {
-      step = pstep;
-      nst.boundary = 0;
-      return 0;
-    }
-    nst.boundary = 1;
-    if (step < 0.) step = 0.;
-  }
-  const double push = step + 1E-6;
-  const V3 np{ld.x * push + lp.x, ld.y * push + lp.y, ld.z * push + lp.z};
-  if (next != -1) {
-    const int nv = g.Daughter(db + next);
-    Xf x;
-    LoadXf(g.Pv(nv), x);
-    LocatePoint<D, M>(g, nv, ApplyGeneric(x, np), nst, false, mixed);
-    return exact;
-  }
-  Relocate<D, M>(g, np, nst, mixed);
-  if (abbox) {
-    while (nst.Top() == cv) nst.Pop();
-  }
-  return exact;
-}
-
-// SimpleNavigator::FindNextBoundaryAndStep for baskets
+// One step of a track up to its relocation: the step length, the state's
+// boundary flag, and where the track goes on (the state is complete when the
+// target is nowhere).  `exact` is raised if the ABBox walk took the sorted
+// order.  `vol` is the current volume; basket form: of the basket's first
+// track.
+//
+// kWayAbbox, kWaySimple: FindNextBoundaryAndStep of the two navigators.
+// kWayBasket: SimpleNavigator::FindNextBoundaryAndStep for baskets
 // (navigation/SimpleNavigator.h:638-743), for one track of a basket whose
 // current volume is `vol` (the top of the basket's first state, :672): the
 // track's own TopMatrix (:660-667); the volume's DistanceToOut with pstep as
@@ -673,55 +850,118 @@ VGA_NAV int FindNextBoundaryAndStep(const NavDev &g, V3 gp, V3 gd, const DPath<D
 // distance > pstep -> physics step off boundary (:708-713); otherwise push
 // by 1e-9 and LocatePoint into the daughter or RelocatePointFromPath
 // (:715-740).
-template <int D, uint32_t M = kAllShapes>
-VGA_NAV void FindNextBoundaryAndStepBasket(const NavDev &g, V3 gp, V3 gd, const DPath<D> &cur, DPath<D> &nst,
-                                           double pstep, double &step, int vol) {
-  const Xf m = TopMatrix(g, cur);
-  const V3 lp = ApplyGeneric(m, gp);
-  const V3 ld = Rotate(m, gd);
-  const PlacedRec &C = g.Pv(vol);
-  step = DDistOut<M>(C.type, g.params + C.param_off, lp, ld, pstep);
+template <int D, uint32_t M, int Way>
+VGA_NAV Target StepTo(const NavDev &g, V3 gp, V3 gd, DPath<D> &nst, double pstep, double &step, int vol, int &exact) {
+  const Target nowhere{-1, -1, V3{0., 0., 0.}, false};
+  V3 lp, ld;
+  {
+    const Xf m = TopMatrix(g, nst);
+    lp = ApplyGeneric(m, gp);
+    ld = Rotate(m, gd);
+  }
+  const Head C = LoadHead(g, vol);
   int next = -1;
-  for (int k = C.dbegin; k < C.dend; ++k) {
-    const double dd = PlacedDistIn<M>(g, g.Daughter(k), lp, ld, step);
-    if (dd < step) {
-      step = dd;
-      next = k - C.dbegin;
+  step = NDistOut<M>(g, vol, C, lp, ld, pstep);
+  if constexpr (Abbox(Way)) {
+    if (step < 0.) step = kInfinity;
+    if (C.nd > 0) exact += Candidates<M, Way>(g, C, lp, ld, step, next);
+    if (step > pstep) {
+      step = pstep;
+      nst.boundary = 0;
+      return nowhere;
     }
+    nst.boundary = 1;
+    if (step > 1E30) {
+      step = 0;
+      nst.Pop();
+      return nowhere;
+    }
+  } else {
+    if (Way == kWaySimple && step <= 0.) step = kInfinity;
+    if (C.nd > 0) Candidates<M, Way>(g, C, lp, ld, step, next);
+    if (Way == kWaySimple && step == kInfinity && pstep > 0.) {
+      step = 0;
+      nst.Pop();
+      nst.boundary = 1;
+      return nowhere;
+    }
+    if (step > pstep) {
+      step = pstep;
+      nst.boundary = 0;
+      return nowhere;
+    }
+    nst.boundary = 1;
   }
-  nst = cur;
-  if (step > pstep) {
-    step = pstep;
-    nst.boundary = 0;
-    return;
-  }
-  nst.boundary = 1;
-  const double push = step + 1E-9;
+  if (Way != kWayBasket && step < 0.) step = 0.;
+  const double push = step + (Way == kWayBasket ? 1E-9 : 1E-6);
   const V3 np{ld.x * push + lp.x, ld.y * push + lp.y, ld.z * push + lp.z};
-  if (next > -1) {
-    const int nv = g.Daughter(C.dbegin + next);
-    Xf x;
-    LoadXf(g.Pv(nv), x);
-    LocatePoint<D, M>(g, nv, ApplyGeneric(x, np), nst, false);
-    return;
-  }
-  Relocate<D, M>(g, np, nst);
+  if (next != -1) return Into(g, g.Daughter(C.dbegin + next), np, nst);
+  return Relocate<D, M>(g, np, nst);
 }
 
-template <int D, uint32_t M = kAllShapes>
+// The rest of the step: descend into the target; the ABBox navigator leaves a
+// volume that a relocation found again (`vol`, the volume before the step).
+template <int D, uint32_t M, int Way>
+VGA_NAV void Arrive(const NavDev &g, const Target &t, int vol, DPath<D> &nst) {
+  Descend<D, M>(g, t, nst);
+  if (Abbox(Way) && t.down)
+    while (nst.Top() == vol) nst.Pop();
+}
+
+// FindNextBoundaryAndStep on the state `nst` in place.
+template <int D, uint32_t M, int Way>
+VGA_NAV void FindNextBoundaryAndStep(const NavDev &g, V3 gp, V3 gd, DPath<D> &nst, double pstep, double &step,
+                                     int vol) {
+  int exact = 0;
+  const Target t = StepTo<D, M, Way>(g, gp, gd, nst, pstep, step, vol, exact);
+  Arrive<D, M, Way>(g, t, vol, nst);
+}
+
+// ABBoxNavigator::GetSafety: the smallest of the volume's SafetyToOut and
+// its daughters' SafetyToIn.  Where the index says that every daughter's
+// SafetyToIn is at least kSafetyShare of the point's distance from its extent
+// in each coordinate, daughters farther than the least safety found so far
+// allows are left out.
+constexpr float kSafetyShare = 0.7f;  // a box turned about z: 1 / sqrt(2)
+template <int D, uint32_t M>
 VGA_NAV double GetSafety(const NavDev &g, V3 gp, const DPath<D> &cur) {
   const Xf m = TopMatrix(g, cur);
   const V3 lp = ApplyGeneric(m, gp);
-  const PlacedRec &C = g.Pv(cur.Top());
-  double safety = DSafeOut<M>(C.type, g.params + C.param_off, lp);
-  for (int k = C.dbegin; k < C.dend; ++k) {
-    const PlacedRec &r = g.Pv(g.Daughter(k));
-    Xf x;
-    LoadXf(r, x);
-    const double t = DSafeIn<M>(r.type, g.params + r.param_off, XfPointRt(x, r.xfkind, lp));
+  const int cv = cur.Top();
+  const Head C = LoadHead(g, cv);
+  double safety = NSafeOut<M>(g, cv, C, lp);
+  if (C.nd <= 0) return safety;
+  Meet near(g, C.code, C.index, C.nd, Finite(lp));
+  if (near.index && !near.index->safe) near.index = nullptr;
+  const F3 p{(float)lp.x, (float)lp.y, (float)lp.z};
+  float reach = near.index ? near.index->first : 0.f;
+  near.Around(p, reach);
+  int w = 0;
+  uint64_t todo = near.Mask(g, 0), seen = todo;
+  while (true) {
+    if (!todo) {
+      if (++w < near.words) {
+        todo = near.Mask(g, w);  // (a daughter seen before changes nothing)
+        continue;
+      }
+      // All seen, all nearer ones seen, or no number to compare with.
+      if (!near.index || safety <= (double)(kSafetyShare * reach) || !(reach < 1e30f) ||
+          (near.words == 1 && seen == near.Full(0)))
+        return safety;
+      reach = safety < (double)(2.f * reach) ? (float)(safety * 1.5) + 1e-3f : 4.f * reach;
+      near.Around(p, reach);
+      w = 0;
+      const uint64_t all = near.Mask(g, 0);
+      todo = all & ~seen;
+      seen = all;
+      continue;
+    }
+    const int id = g.Daughter(C.dbegin + 64 * w + __builtin_ctzll(todo));
+    todo &= todo - 1;
+    const Head h = LoadHead(g, id);
+    const double t = NSafeIn<M>(g, id, h, XfPointRt(LoadXf(g, id, h.code), KindOf(h.code), lp));
     safety = Min(safety, t);
   }
-  return safety;
 }
 
 // The TraceTrack loop for one track (TraceTrack.cpp:170-220): locate from
@@ -729,77 +969,87 @@ VGA_NAV double GetSafety(const NavDev &g, V3 gp, const DPath<D> &cur) {
 // state leaves the world or max_steps steps were taken.  Returns the number
 // of steps; p ends at the final point.  The hash folds
 // (new top id + 1) * 2 + boundary after every step.
-template <int D, bool ExactOnly = false, uint32_t M = kAllShapes, bool Mixed = false>
-VGA_NAV int TraceOne(const NavDev &g, V3 &p, V3 d, double pstep, int kind, int max_steps, double &dist, uint64_t &h,
+template <int D, uint32_t M, int Way>
+VGA_NAV int TraceOne(const NavDev &g, V3 &p, V3 d, double pstep, int max_steps, double &dist, uint64_t &h,
                      int &nexact) {
-  DPath<D> cur, nst;
+  DPath<D> cur;
   cur.Clear();
-  LocatePoint<D, M>(g, g.world, p, cur, true, Mixed);
-  int k = 0;
+  Target t = FromWorld<D, M>(g, p, cur);
+  int k = -1, vol = -1;
   nexact = 0;
   dist = 0;
   h = 1469598103934665603ULL;
-  while (cur.level > 0 && k < max_steps) {
-    double step;
-    nexact += FindNextBoundaryAndStep<D, ExactOnly, M, Mixed>(g, p, d, cur, nst, pstep, step, kind);
-    dist += step;
-    const double s = step + 1E-6;
-    p = V3{p.x + d.x * s, p.y + d.y * s, p.z + d.z * s};
-    cur = nst;
-    const uint64_t v = (uint64_t)(uint32_t)(cur.Top() + 1) * 2ULL + (cur.boundary ? 1ULL : 0ULL);
-    h = (h ^ v) * 1099511628211ULL;
-    ++k;
+  double step = 0;
+  while (true) {
+    Arrive<D, M, Way>(g, t, vol, cur);
+    if (++k > 0) {
+      dist += step;
+      const double s = step + 1E-6;
+      p = V3{p.x + d.x * s, p.y + d.y * s, p.z + d.z * s};
+      const uint64_t v = (uint64_t)(uint32_t)(cur.Top() + 1) * 2ULL + (cur.boundary ? 1ULL : 0ULL);
+      h = (h ^ v) * 1099511628211ULL;
+    }
+    if (!(cur.level > 0 && k < max_steps)) return k;
+    vol = cur.Top();
+    t = StepTo<D, M, Way>(g, p, d, cur, pstep, step, vol, nexact);
   }
-  return k;
+}
+
+// Tracks per wave of a navigation launch over n tracks, as a power of two: 64
+// where that gives the chip two waves per SIMD, fewer for small baskets.  A
+// wave runs as long as its slowest lane and through the code of every volume
+// type that its lanes meet, so spreading few tracks over idle SIMDs shortens
+// every step: 1,000 nested tracks 4.3 -> 1.9 ms, 4,000 2.3 ms with 1,024
+// waves, 1.50 with 2,048 and 2.71 with 4,096; one step of 65,537 tracks with
+// its locate and safety 85, 86 and 105 us.
+constexpr uint64_t kNavWaves = 2048;
+inline int LanesShift(uint64_t n) {
+  int s = 0;
+  while (s < 6 && (n >> s) > kNavWaves) ++s;
+  return s;
+}
+// The lane's track under that shift (waves of 64 threads); n or more: none.
+VGA_NAV uint64_t TrackOf(uint64_t thread, int shift, uint64_t n) {
+  const uint64_t lane = thread & 63;
+  return (lane >> shift) ? n : ((thread >> 6) << shift) + lane;
+}
+
+// The navigator's view of an uploaded geometry.
+inline NavDev DeviceNav(const vg_geometry *g) {
+  return NavDev{g->d_nav,
+                g->d_placed,
+                g->d_params,
+                g->d_slot_aabb,
+                g->d_dindex,
+                g->d_dmasks,
+                g->world,
+                (int32_t)g->placed.size(),
+                (int32_t)g->daughters.size(),
+                (int32_t)g->dindex.size(),
+                (int32_t)g->dmasks.size()};
+}
+
+// Calls f(D, M) with the path depth D (4, 8 or 16) that holds the geometry
+// and the smallest shape set M of three that holds its shapes (both
+// std::integral_constant).
+template <class F>
+void WithVariant(const vg_geometry *g, F f) {
+  const uint32_t beyond = g->type_mask & ~kBasicShapes;
+  auto shapes = [&](auto depth) {
+    if (beyond == 0)
+      f(depth, std::integral_constant<uint32_t, kBasicShapes>{});
+    else if (beyond == kPhiTube)
+      f(depth, std::integral_constant<uint32_t, kBasicShapes | kPhiTube>{});
+    else
+      f(depth, std::integral_constant<uint32_t, kAllShapes>{});
+  };
+  if (g->max_depth <= 4)
+    shapes(std::integral_constant<int, 4>{});
+  else if (g->max_depth <= 8)
+    shapes(std::integral_constant<int, 8>{});
+  else
+    shapes(std::integral_constant<int, 16>{});
 }
 
 }  // namespace nav
 }  // namespace vga
-
-// Launches KERNEL<D, M, MX> with the path depth D (8 or 16) that holds the
-// geometry, the shape set M (the basic shapes only when the geometry uses
-// nothing else, all shapes otherwise) and MX = the mixed-precision
-// navigator (MIXED, a run-time bool).
-#define VGA_NAV_VARIANTS_MX(G, MIXED, KERNEL, ...)                                        \
-  do {                                                                                    \
-    const bool light_ = ((G)->type_mask & ~::vga::nav::kBasicShapes) == 0;                \
-    const bool d8_ = (G)->max_depth <= 8;                                                 \
-    if (MIXED) {                                                                          \
-      if (d8_ && light_)                                                                  \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kBasicShapes, true>), __VA_ARGS__);     \
-      else if (d8_)                                                                       \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kAllShapes, true>), __VA_ARGS__);       \
-      else if (light_)                                                                    \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kBasicShapes, true>), __VA_ARGS__);    \
-      else                                                                                \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kAllShapes, true>), __VA_ARGS__);      \
-    } else {                                                                              \
-      if (d8_ && light_)                                                                  \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kBasicShapes, false>), __VA_ARGS__);    \
-      else if (d8_)                                                                       \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kAllShapes, false>), __VA_ARGS__);      \
-      else if (light_)                                                                    \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kBasicShapes, false>), __VA_ARGS__);   \
-      else                                                                                \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kAllShapes, false>), __VA_ARGS__);     \
-    }                                                                                     \
-  } while (0)
-
-// Launches KERNEL<D, M> with the path depth D (8 or 16) that holds the
-// geometry and the shape set M: the basic shapes only when the geometry uses
-// nothing else, all shapes otherwise.
-#define VGA_NAV_VARIANTS(G, KERNEL, ...)                                          \
-  do {                                                                            \
-    const bool light_ = ((G)->type_mask & ~::vga::nav::kBasicShapes) == 0;        \
-    if ((G)->max_depth <= 8) {                                                    \
-      if (light_)                                                                 \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kBasicShapes>), __VA_ARGS__);   \
-      else                                                                        \
-        hipLaunchKernelGGL((KERNEL<8, ::vga::nav::kAllShapes>), __VA_ARGS__);     \
-    } else {                                                                      \
-      if (light_)                                                                 \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kBasicShapes>), __VA_ARGS__);  \
-      else                                                                        \
-        hipLaunchKernelGGL((KERNEL<16, ::vga::nav::kAllShapes>), __VA_ARGS__);    \
-    }                                                                             \
-  } while (0)

@@ -48,12 +48,6 @@ using namespace nav;
 using Clock = std::chrono::steady_clock;
 
 constexpr int kServeBlock = 128;
-// The world volume's daughter boxes are staged in LDS by the step kernel
-// when they take at most this many bytes.
-constexpr size_t kServeBoxLds = 8192;
-// ... and, with the mixed navigator, their FP32 bound records (144 bytes
-// each) when those take at most this many bytes more.
-constexpr size_t kServeBoundLds = 9216;
 constexpr int kMaxStreams = 2;
 constexpr int kMaxSegs = 4096;  // requests merged into one launch at most
 
@@ -95,7 +89,8 @@ __global__ __launch_bounds__(kServeBlock) void ServeLocateKernel(const NavDev g,
   const uint64_t s = offset + i;
   DPath<D> p;
   p.Clear();
-  LocatePoint<D, M>(g, g.world, V3{a.x[s], a.y[s], a.z[s]}, p, true);
+  const Target t = FromWorld<D, M>(g, V3{a.x[s], a.y[s], a.z[s]}, p);
+  Descend<D, M>(g, t, p);
   a.level[s] = p.level;
   a.boundary[s] = 0;
   for (int l = 0; l < a.depth; ++l) a.path[(uint64_t)l * a.cap + s] = l < D ? p.Get(l) : -1;
@@ -105,47 +100,20 @@ __global__ __launch_bounds__(kServeBlock) void ServeLocateKernel(const NavDev g,
 }
 
 // One step of every track of every segment; a track outside the world
-// (level 0) stays where it is with step 0.  Tiles of kServeBlock tracks are
-// numbered across segments; each block finds its segment by binary search.
-template <int D, uint32_t M, bool MX>
+// (level 0) stays where it is with step 0.  Tiles of kServeBlock lanes
+// ((kServeBlock / 64) << shift tracks, LanesShift) are numbered across
+// segments; each block finds its segment by binary search.
+template <int D, uint32_t M, int Way>
 __global__ __launch_bounds__(kServeBlock) void ServeStepKernel(const NavDev g, const Arena a,
                                                                const Seg *__restrict__ segs, int nseg, uint64_t ntiles,
-                                                               double pstep, int kind, int stage_lo, int stage_hi,
-                                                               int stage_bounds) {
-  // The world volume's daughter-slot boxes in LDS (as the trace kernel
-  // stages them; none when stage_lo == stage_hi), and in the mixed kernel
-  // their FP32 bound records after them.
-  extern __shared__ __align__(16) float serve_boxes[];
-  NavDev gl = g;
-  if (stage_hi > stage_lo) {  // uniform over the grid
-    const int nf = 8 * (stage_hi - stage_lo);
-    const float *src = g.slot_box + 8 * (size_t)stage_lo;
-    for (int j = threadIdx.x; j < nf; j += kServeBlock) serve_boxes[j] = src[j];
-    __syncthreads();
-    gl.lds_box = serve_boxes;
-    gl.lds_lo = stage_lo;
-    gl.lds_hi = stage_hi;
-    if constexpr (MX) {
-      if (stage_bounds) {  // uniform over the grid: the same daughters' FP32 bound records
-        constexpr int kRec = (int)(sizeof(B32) / sizeof(uint32_t));
-        uint32_t *dst = reinterpret_cast<uint32_t *>(serve_boxes + nf);
-        const int nr = kRec * (stage_hi - stage_lo);
-        for (int j = threadIdx.x; j < nr; j += kServeBlock) {
-          const int slot = stage_lo + j / kRec;
-          dst[j] = reinterpret_cast<const uint32_t *>(g.b32 + g.daughters[slot])[j % kRec];
-        }
-        __syncthreads();
-        gl.lds_bound = reinterpret_cast<const B32 *>(dst);
-      }
-    }
-  }
+                                                               double pstep, int shift) {
   const uint64_t tile = blockIdx.x;
   if (tile >= ntiles) return;
   const Seg sg = segs[FindSeg(segs, nseg, tile)];
-  const uint64_t i = (tile - sg.tile_begin) * kServeBlock + threadIdx.x;
+  const uint64_t i = TrackOf((tile - sg.tile_begin) * kServeBlock + threadIdx.x, shift, sg.n);
   if (i >= sg.n) return;
   const uint64_t s = sg.offset + i;
-  DPath<D> cur, nst;
+  DPath<D> cur;
   cur.level = a.level[s];
   cur.boundary = a.boundary[s];
 #pragma unroll
@@ -157,18 +125,18 @@ __global__ __launch_bounds__(kServeBlock) void ServeStepKernel(const NavDev g, c
   V3 p{a.x[s], a.y[s], a.z[s]};
   const V3 d{a.dx[s], a.dy[s], a.dz[s]};
   double step;
-  FindNextBoundaryAndStep<D, false, M, MX>(gl, p, d, cur, nst, pstep, step, kind);
+  FindNextBoundaryAndStep<D, M, Way>(g, p, d, cur, pstep, step, cur.Top());
   const double sp = step + 1E-6;
   p = V3{p.x + d.x * sp, p.y + d.y * sp, p.z + d.z * sp};
   a.x[s] = p.x;
   a.y[s] = p.y;
   a.z[s] = p.z;
   a.step[s] = step;
-  a.level[s] = nst.level;
-  a.boundary[s] = nst.boundary;
-  for (int l = 0; l < a.depth; ++l) a.path[(uint64_t)l * a.cap + s] = l < D ? nst.Get(l) : -1;
+  a.level[s] = cur.level;
+  a.boundary[s] = cur.boundary;
+  for (int l = 0; l < a.depth; ++l) a.path[(uint64_t)l * a.cap + s] = l < D ? cur.Get(l) : -1;
   a.nsteps[s] += 1;
-  const uint64_t v = (uint64_t)(uint32_t)(nst.Top() + 1) * 2ULL + (nst.boundary ? 1ULL : 0ULL);
+  const uint64_t v = (uint64_t)(uint32_t)(cur.Top() + 1) * 2ULL + (cur.boundary ? 1ULL : 0ULL);
   a.hash[s] = (a.hash[s] ^ v) * 1099511628211ULL;
 }
 
@@ -180,9 +148,6 @@ using namespace vga;
 struct vg_server {
   const vg_geometry *g = nullptr;
   NavDev dev{};
-  int stage_lo = 0, stage_hi = 0;  // world daughter slots staged in LDS by the step kernel
-  int stage_bounds = 0;            // 1: their FP32 bound records too (mixed navigator)
-  size_t box_bytes = 0;            // LDS bytes of the step kernel
   Arena a{};
   int navigator = VG_NAV_ABBOX;
   double pstep = 0;
@@ -254,13 +219,16 @@ void StartLaunch(vg_server *s, int k) {
   s->pending.swap(keep);
   s->npending.store((int64_t)s->pending.size(), std::memory_order_release);
   if (take.empty()) return;
-  uint64_t tiles = 0;
+  uint64_t tiles = 0, tracks = 0;
+  for (int64_t r : take) tracks += s->baskets[s->requests[r].basket].n;
+  const int shift = LanesShift(tracks);
+  const uint64_t per = (uint64_t)(kServeBlock / 64) << shift;
   int nseg = 0;
   for (int64_t r : take) {
     const auto &b = s->baskets[s->requests[r].basket];
     if (b.n == 0) continue;
     s->h_segs[k][nseg] = Seg{b.offset, b.n, tiles};
-    tiles += (b.n + kServeBlock - 1) / kServeBlock;
+    tiles += (b.n + per - 1) / per;
     s->track_steps += b.n;
     ++nseg;
   }
@@ -269,9 +237,17 @@ void StartLaunch(vg_server *s, int k) {
     rc = CheckHip(hipMemcpyAsync(s->d_segs[k], s->h_segs[k], nseg * sizeof(Seg), hipMemcpyHostToDevice, s->stream[k]),
                   "serve segment upload");
     if (!rc) {
-      VGA_NAV_VARIANTS_MX(s->g, s->navigator == VG_NAV_ABBOX_MIXED, ServeStepKernel, dim3((unsigned)tiles),
-                          dim3(kServeBlock), s->box_bytes, s->stream[k], s->dev, s->a, s->d_segs[k], nseg, tiles,
-                          s->pstep, s->navigator, s->stage_lo, s->stage_hi, s->stage_bounds);
+      const dim3 blocks((unsigned)tiles), threads(kServeBlock);
+      if (s->navigator == VG_NAV_SIMPLE)
+        WithVariant(s->g, [&](auto D, auto M) {
+          hipLaunchKernelGGL((ServeStepKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, s->stream[k],
+                             s->dev, s->a, s->d_segs[k], nseg, tiles, s->pstep, shift);
+        });
+      else
+        WithVariant(s->g, [&](auto D, auto M) {
+          hipLaunchKernelGGL((ServeStepKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, s->stream[k],
+                             s->dev, s->a, s->d_segs[k], nseg, tiles, s->pstep, shift);
+        });
       rc = CheckHip(hipGetLastError(), "serve step launch");
     }
   }
@@ -401,7 +377,10 @@ int Open(vg_server *s, uint64_t n, const double *const src[6], int64_t *basket) 
     rc = CheckHip(hipMemcpyAsync(dst[i] + off, src[i], n * 8, hipMemcpyHostToDevice, s->ustream), "basket upload");
   if (!rc && n) {
     const unsigned blocks = (unsigned)((n + kServeBlock - 1) / kServeBlock);
-    VGA_NAV_VARIANTS(s->g, ServeLocateKernel, dim3(blocks), dim3(kServeBlock), 0, s->ustream, s->dev, s->a, off, n);
+    WithVariant(s->g, [&](auto D, auto M) {
+      hipLaunchKernelGGL((ServeLocateKernel<D.value, M.value>), dim3(blocks), dim3(kServeBlock), 0, s->ustream,
+                         s->dev, s->a, off, n);
+    });
     rc = CheckHip(hipGetLastError(), "basket locate");
   }
   if (!rc) rc = CheckHip(hipStreamSynchronize(s->ustream), "basket open sync");
@@ -474,22 +453,7 @@ int vg_server_create(const vg_geometry *g, uint64_t hbm_budget_bytes, int32_t na
   s->g = g;
   s->navigator = navigator;
   s->pstep = pstep;
-  s->dev = NavDev{g->d_placed, g->d_params, g->d_daughters, g->d_aabb, g->d_b32, g->d_b32side, g->d_slot_aabb,
-                  g->world,    (int32_t)g->placed.size(), (int32_t)g->daughters.size(), 0};
-  if (g->world >= 0) {
-    const PlacedRec &w = g->placed[g->world];
-    const size_t bytes = 8 * sizeof(float) * (size_t)(w.dend - w.dbegin);
-    if (bytes > 0 && bytes <= kServeBoxLds) {
-      s->stage_lo = w.dbegin;
-      s->stage_hi = w.dend;
-      s->box_bytes = bytes;
-      const size_t bound_bytes = sizeof(B32) * (size_t)(w.dend - w.dbegin);
-      if (navigator == VG_NAV_ABBOX_MIXED && g->d_b32 && bound_bytes <= kServeBoundLds) {
-        s->stage_bounds = 1;
-        s->box_bytes += bound_bytes;
-      }
-    }
-  }
+  s->dev = DeviceNav(g);
   rc = CheckHip(hipMalloc(&s->mem, cap * SlotBytes(depth)), "hipMalloc(serve arena)");
   if (!rc) {
     char *m = static_cast<char *>(s->mem);

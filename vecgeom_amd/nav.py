@@ -24,7 +24,7 @@ from . import capi
 
 ABBOX = 0
 SIMPLE = 1
-ABBOX_MIXED = 2  # ABBox navigator with the FP32 daughter filter (same results)
+ABBOX_MIXED = 2  # the ABBox navigator (its daughters are preselected in FP32 under either name)
 SIMPLE_BASKET = 3  # SimpleNavigator's basket step: one current volume for the whole basket
 MAX_DEPTH = 16
 HASH_SEED = 1469598103934665603

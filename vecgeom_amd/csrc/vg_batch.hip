@@ -56,7 +56,8 @@ constexpr int kBatchBlock = 256;
 struct TaskDev {
   int32_t type, query, xfkind, in_type;
   int32_t param_off, vec_ok;
-  int32_t param_len, pad;  // parameter block length (doubles)
+  int32_t param_len;   // parameter block length (doubles)
+  int32_t tile_items;  // items per tile
   uint64_t n, tile_begin;
   const void *x, *y, *z, *dx, *dy, *dz;
   const double *sm;
@@ -335,17 +336,34 @@ constexpr int ClassOf(int type) {
 // Items per lane of class c when the batch asks for `it`: the light class
 // takes it as given, the compute-heavy classes at most 2.
 constexpr int ClassIT(int c, int it) { return Base(c) == 0 ? it : (it < 2 ? it : 2); }
+// ... and 1 in a heavy class whose `items` queries would not give each CU
+// kHeavyTiles tiles: such a launch lasts as long as its longest lane, and a
+// second item on that lane doubles it.
+constexpr uint64_t kHeavyTiles = 4 * 256;
+constexpr int RunIT(int c, int it, uint64_t items) {
+  return Base(c) != 0 && items < kHeavyTiles * kBatchBlock * 2 ? 1 : ClassIT(c, it);
+}
 
 // The Polyhedron's distance tasks in the staged class run with lane refill
-// (vg_walk.hpp) over tiles kWalkTileMul times longer, so that each wave
-// refills its lanes from 4 * 64 * IT queries.  (The Polycone's measured
-// slower as walks, DistanceToIn and DistanceToOut alike.)
+// (vg_walk.hpp) over longer tiles, so that each wave refills its lanes from
+// up to 4 * 64 * IT queries; a task with fewer than kWalkQueries queries for
+// each of them takes shorter tiles, down to one query a lane, and so spreads
+// over more waves.  (With the single item per lane of RunIT: the twelve
+// shapes' 72 tasks of 4,099 points each 128 -> 77 us, the staged class's
+// kernel 104 us of the 128.)  (The Polycone's measured slower as walks,
+// DistanceToIn and DistanceToOut alike.)
 constexpr int kWalkTileMul = 4;
+constexpr uint64_t kWalkQueries = 64 * 1024;
 constexpr bool WalkTask(int type, int query) {
   return type == VG_POLYHEDRON && (query == kQDistIn || query == kQDistOut || query == kQPlacedDistOut);
 }
-constexpr uint64_t TileItems(int c, int it, int type, int query) {
-  return (uint64_t)kBatchBlock * ClassIT(c, it) * ((Base(c) == kStagedClass && WalkTask(type, query)) ? kWalkTileMul : 1);
+// Items per tile of a task of n queries in a class that runs `it` per lane.
+constexpr int TileItems(int c, int it, int type, int query, uint64_t n) {
+  const int most = kWalkTileMul * it;
+  const uint64_t lane = n / kWalkQueries;
+  return kBatchBlock *
+         (Base(c) == kStagedClass && WalkTask(type, query) ? (lane < 1 ? 1 : lane < (uint64_t)most ? (int)lane : most)
+                                                           : it);
 }
 
 // The four short queries of a shape (CheapQuery), FP64 or FP32 storage.
@@ -569,7 +587,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(Cla
       __syncthreads();
       blk = stage;
       if (WalkTask(t.type, t.query)) {  // uniform over the workgroup
-        const uint64_t per = TileItems(CLS, IT, t.type, t.query), first = (tile - t.tile_begin) * per;
+        const uint64_t per = t.tile_items, first = (tile - t.tile_begin) * per;
         if (t.query == kQDistIn) {
           RunTileWalk<PolyhedronS, PolyhedronS::DistInOps, false, MX>(t, stage, first, per);
         } else if (t.query == kQDistOut) {
@@ -705,11 +723,12 @@ int TaskClass(const TaskDev &t) {
 void Schedule(vg_batch *b) {
   for (int c = 0; c < kClasses; ++c) {
     uint64_t tile = 0;
+    const int it = RunIT(c, b->it, b->class_items[c]);
     for (int k = b->first[c]; k < b->first[c + 1]; ++k) {
       TaskDev &x = b->host[k];
-      const uint64_t per = TileItems(c, b->it, x.type, x.query);
+      x.tile_items = TileItems(c, it, x.type, x.query, x.n);
       x.tile_begin = tile;
-      tile += (x.n + per - 1) / per;
+      tile += (x.n + x.tile_items - 1) / x.tile_items;
     }
     b->ntiles[c] = tile;
   }
@@ -724,7 +743,7 @@ void LaunchClass(const vg_batch *b, unsigned grid, hipStream_t s) {
 
 template <int CLS>
 void LaunchIT(const vg_batch *b, unsigned grid, hipStream_t s) {
-  const int it = ClassIT(CLS, b->it);
+  const int it = RunIT(CLS, b->it, b->class_items[CLS]);
   if (it == 1)
     LaunchClass<1, CLS>(b, grid, s);
   else if (it == 2)
@@ -962,12 +981,15 @@ int ScratchPtr(TaskDev **out) {
 }
 
 template <int CLS>
-void LaunchNoAlloc(const TaskDev *tasks, int ntasks, uint64_t ntiles, int stage_len, const double *params,
+void LaunchNoAlloc(int it, const TaskDev *tasks, int ntasks, uint64_t ntiles, int stage_len, const double *params,
                    hipStream_t s) {
-  constexpr int IT = ClassIT(CLS, 2);
   const size_t lds = Base(CLS) == kStagedClass ? (size_t)stage_len * sizeof(double) : 0;
-  hipLaunchKernelGGL((BatchKernel<IT, CLS>), dim3((unsigned)ntiles), dim3(kBatchBlock), lds, s, tasks, ntasks, ntiles,
-                     params);
+  if (it == 1)
+    hipLaunchKernelGGL((BatchKernel<1, CLS>), dim3((unsigned)ntiles), dim3(kBatchBlock), lds, s, tasks, ntasks, ntiles,
+                       params);
+  else
+    hipLaunchKernelGGL((BatchKernel<2, CLS>), dim3((unsigned)ntiles), dim3(kBatchBlock), lds, s, tasks, ntasks, ntiles,
+                       params);
 }
 
 }  // namespace
@@ -993,16 +1015,18 @@ int vg_batch_run_noalloc(const vg_geometry *g, const vg_query_task *tasks, int32
   }
   if (n == 0) return VG_OK;
   std::stable_sort(host, host + n, [](const TaskDev &a, const TaskDev &c) { return TaskClass(a) < TaskClass(c); });
-  int first[kClasses + 1];
+  int first[kClasses + 1], run_it[kClasses];
   uint64_t ntiles[kClasses];
   int stage_len = 0;
   for (int c = 0, k = 0; c < kClasses; ++c) {
     first[c] = k;
-    uint64_t tile = 0;
+    uint64_t tile = 0, items = 0;
+    for (int j = k; j < n && TaskClass(host[j]) == c; ++j) items += host[j].n;
+    run_it[c] = RunIT(c, 2, items);
     for (; k < n && TaskClass(host[k]) == c; ++k) {
-      const uint64_t per = TileItems(c, 2, host[k].type, host[k].query);
+      host[k].tile_items = TileItems(c, run_it[c], host[k].type, host[k].query, host[k].n);
       host[k].tile_begin = tile;
-      tile += (host[k].n + per - 1) / per;
+      tile += (host[k].n + host[k].tile_items - 1) / host[k].tile_items;
       if (Base(c) == kStagedClass) stage_len = std::max(stage_len, host[k].param_len);
     }
     ntiles[c] = tile;
@@ -1017,16 +1041,16 @@ int vg_batch_run_noalloc(const vg_geometry *g, const vg_query_task *tasks, int32
     const TaskDev *tt = dev + first[c];
     const int cnt = first[c + 1] - first[c];
     switch (c) {
-      case 0: LaunchNoAlloc<0>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 1: LaunchNoAlloc<1>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 2: LaunchNoAlloc<2>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 3: LaunchNoAlloc<3>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 4: LaunchNoAlloc<4>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 5: LaunchNoAlloc<5>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 6: LaunchNoAlloc<6>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 7: LaunchNoAlloc<7>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      case 8: LaunchNoAlloc<8>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
-      default: LaunchNoAlloc<9>(tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 0: LaunchNoAlloc<0>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 1: LaunchNoAlloc<1>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 2: LaunchNoAlloc<2>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 3: LaunchNoAlloc<3>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 4: LaunchNoAlloc<4>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 5: LaunchNoAlloc<5>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 6: LaunchNoAlloc<6>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 7: LaunchNoAlloc<7>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      case 8: LaunchNoAlloc<8>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
+      default: LaunchNoAlloc<9>(run_it[c], tt, cnt, ntiles[c], stage_len, g->d_params, s); break;
     }
     rc = CheckHip(hipGetLastError(), "no-allocation batch launch");
   }

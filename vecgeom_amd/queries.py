@@ -5,9 +5,53 @@ Each function mirrors a VPlacedVolume SOA3D virtual
 triples of 1-D float64 CUDA tensors (SOA3D); outputs are new CUDA tensors
 unless `out` is given.  Work is enqueued on torch's current stream.
 """
+import ctypes
+import importlib.util
+import os
+
 import torch
 
 from . import capi
+
+# Output types and argument lists of the native front (csrc/py_queries.cpp).
+_U8, _I32, _F64 = 0, 1, 2
+_POINTS, _RAYS, _RAYS_NEXT, _NORMAL, _RAYS_NORMAL = range(5)
+_front = None
+_address = {}
+
+
+def _load_front():
+    """Loads the native front and the entry points' addresses once; raises if
+    it is not built."""
+    global _front
+    path = os.path.join(capi.HERE, "lib", "_vgq.so")
+    if not os.path.exists(path):
+        raise RuntimeError(f"{path} is missing: build it with __graft_entry__.build()")
+    lib = capi.lib()
+    for name in ("vg_contains", "vg_inside", "vg_distance_to_in", "vg_distance_to_out", "vg_placed_distance_to_out",
+                 "vg_safety_to_in", "vg_safety_to_out", "vg_unplaced_contains", "vg_normal",
+                 "vg_distance_to_out_normal"):
+        _address[name] = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+    spec = importlib.util.spec_from_file_location("vecgeom_amd._vgq", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    _front = module.run
+    return _front
+
+
+def _native(name, family, geom, placed, p, d=None, step_max=None, out=None, code=_F64, next_node=None):
+    """The query through the native front: its output, or None where the
+    arguments are not the usual ones (the callers' own checks then say why)."""
+    run = _front or _load_front()
+    handle = geom.handle
+    if handle is None:
+        return None
+    r = run(_address[name], family, handle.value, placed, p, d, step_max, out, code, next_node)
+    if r is None:
+        return None
+    if r[0] != capi.VG_OK:
+        raise RuntimeError(f"{name} failed ({r[0]}): {capi.lib().vg_last_error().decode(errors='replace')}")
+    return r[1]
 
 
 def _stream():
@@ -53,6 +97,9 @@ def _ptrs(p):
 
 
 def contains(geom, placed, p, out=None):
+    r = _native("vg_contains", _POINTS, geom, placed, p, out=out, code=_U8)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     out = _out(out, torch.uint8, n, p[0].device)
     capi.call("vg_contains", geom.handle, int(placed), *_ptrs(p), n, out.data_ptr(), _stream())
@@ -71,6 +118,9 @@ def contains_local(geom, placed, p, out=None):
 
 def unplaced_contains(geom, placed, lp, out=None):
     """UnplacedContains(localPoint) (volumes/PlacedVolume.h:158-160)."""
+    r = _native("vg_unplaced_contains", _POINTS, geom, placed, lp, out=out, code=_U8)
+    if r is not None:
+        return r
     n = _check_soa(lp, "local points")
     out = _out(out, torch.uint8, n, lp[0].device)
     capi.call("vg_unplaced_contains", geom.handle, int(placed), *_ptrs(lp), n, out.data_ptr(), _stream())
@@ -82,6 +132,9 @@ def normal(geom, placed, lp):
     and the shapes' overrides) on local points: returns ((nx, ny, nz) float64,
     uint8 valid).  Box, Tube, Orb, Sphere, Cone, Trd, Trapezoid and Polycone;
     the other shapes raise (their reference Normal asserts)."""
+    r = _native("vg_normal", _NORMAL, geom, placed, lp)
+    if r is not None:
+        return r
     n = _check_soa(lp, "local points")
     dev = lp[0].device
     nrm = tuple(torch.empty(n, dtype=torch.float64, device=dev) for _ in range(3))
@@ -94,6 +147,9 @@ def distance_to_out_normal(geom, placed, lp, ld, step_max=None):
     """The USolids DistanceToOut(point, direction, normal&, convex&, stepMax)
     (volumes/ShapeImplementationHelper.h:277-295) on local rays: returns
     (distance, (nx, ny, nz), uint8 valid, uint8 convex)."""
+    r = _native("vg_distance_to_out_normal", _RAYS_NORMAL, geom, placed, lp, ld, step_max)
+    if r is not None:
+        return r
     n = _check_soa(lp, "local points")
     _check_soa(ld, "local directions", n, lp[0].device)
     dev = lp[0].device
@@ -128,6 +184,9 @@ def scalar(geom, placed, query, point, direction=None, step_max=float("inf")):
 
 
 def inside(geom, placed, p, out=None):
+    r = _native("vg_inside", _POINTS, geom, placed, p, out=out, code=_I32)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     out = _out(out, torch.int32, n, p[0].device)
     capi.call("vg_inside", geom.handle, int(placed), *_ptrs(p), n, out.data_ptr(), _stream())
@@ -135,6 +194,9 @@ def inside(geom, placed, p, out=None):
 
 
 def distance_to_in(geom, placed, p, d, step_max=None, out=None):
+    r = _native("vg_distance_to_in", _RAYS, geom, placed, p, d, step_max, out)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     _check_soa(d, "directions", n, p[0].device)
     out = _out(out, torch.float64, n, p[0].device)
@@ -153,6 +215,9 @@ def distance_to_in_minimize(geom, placed, daughter_index, p, d, inout_dist, inou
 
 
 def distance_to_out(geom, placed, p, d, step_max=None, out=None, next_node=None):
+    r = _native("vg_distance_to_out", _RAYS_NEXT, geom, placed, p, d, step_max, out, _F64, next_node)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     _check_soa(d, "directions", n, p[0].device)
     out = _out(out, torch.float64, n, p[0].device)
@@ -164,6 +229,9 @@ def distance_to_out(geom, placed, p, d, step_max=None, out=None, next_node=None)
 
 
 def placed_distance_to_out(geom, placed, p, d, step_max=None, out=None):
+    r = _native("vg_placed_distance_to_out", _RAYS, geom, placed, p, d, step_max, out)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     _check_soa(d, "directions", n, p[0].device)
     out = _out(out, torch.float64, n, p[0].device)
@@ -174,6 +242,9 @@ def placed_distance_to_out(geom, placed, p, d, step_max=None, out=None):
 
 
 def safety_to_in(geom, placed, p, out=None):
+    r = _native("vg_safety_to_in", _POINTS, geom, placed, p, out=out)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     out = _out(out, torch.float64, n, p[0].device)
     capi.call("vg_safety_to_in", geom.handle, int(placed), *_ptrs(p), n, out.data_ptr(), _stream())
@@ -187,6 +258,9 @@ def safety_to_in_minimize(geom, placed, p, inout):
 
 
 def safety_to_out(geom, placed, p, out=None):
+    r = _native("vg_safety_to_out", _POINTS, geom, placed, p, out=out)
+    if r is not None:
+        return r
     n = _check_soa(p, "points")
     out = _out(out, torch.float64, n, p[0].device)
     capi.call("vg_safety_to_out", geom.handle, int(placed), *_ptrs(p), n, out.data_ptr(), _stream())

@@ -30,7 +30,16 @@ struct BooleanP {
   const double *b;
 };
 
-struct BooleanS {
+// Operand shapes compiled into a Boolean's code (bit t: shape type t): every
+// primitive shape, or all but the Torus.
+constexpr uint32_t kBoolNoTorus = (1u << VG_BOX) | (1u << VG_TUBE) | (1u << VG_ORB) | (1u << VG_SPHERE) |
+                                  (1u << VG_CONE) | (1u << VG_TRD) | (1u << VG_TRAPEZOID) |
+                                  (1u << VG_PARALLELEPIPED) | (1u << VG_PARABOLOID) | (1u << VG_POLYCONE) |
+                                  (1u << VG_POLYHEDRON);
+constexpr uint32_t kBoolAll = kBoolNoTorus | (1u << VG_TORUS);
+
+template <uint32_t M>
+struct BooleanT {
   using P = BooleanP;
   static constexpr int kMaxBooleanIterations = 1000;
   enum { kUnionOp = 0, kIntersectionOp = 1, kSubtractionOp = 2 };
@@ -58,11 +67,13 @@ struct BooleanS {
       case VG_TRAPEZOID: return f(TrapS{}, ParamView<TrapS>::Get(blk));
       case VG_PARALLELEPIPED: return f(ParaS{}, ParamView<ParaS>::Get(blk));
       case VG_PARABOLOID: return f(ParabS{}, ParamView<ParabS>::Get(blk));
-      case VG_TORUS: return f(TorusS{}, ParamView<TorusS>::Get(blk));
+      case VG_TORUS:
+        if constexpr ((M >> VG_TORUS) & 1u) return f(TorusS{}, ParamView<TorusS>::Get(blk));
+        break;
       case VG_POLYCONE: return f(PolyconeS{}, ParamView<PolyconeS>::Get(blk));
       case VG_POLYHEDRON: return f(PolyhedronS{}, ParamView<PolyhedronS>::Get(blk));
-      default: return f(BoxS{}, ParamView<BoxS>::Get(blk));
     }
+    return f(BoxS{}, ParamView<BoxS>::Get(blk));
   }
 
   // The operand's VPlacedVolume virtuals (volumes/PlacedVolume.h:147-250).
@@ -293,6 +304,8 @@ struct BooleanS {
     return Min(safety, safetyright);
   }
 };
+
+using BooleanS = BooleanT<kBoolAll>;
 
 template <>
 struct ParamView<BooleanS> {

@@ -911,8 +911,8 @@ def nav_bench(args, dev, stream, with_cpu):
            "exact_walk_steps": exact, "kernel": "TraceKernel (fused TraceTrack loop)",
            "avg_launch_ms": round(fused_ms, 3), "value": round(total_steps / (fused_ms * 1e-3) / 1e9, 4),
            "unit": "G steps/s", "dtype": "f64"}
-    # The mixed-precision navigator (FP32 filters in the daughter walk and
-    # the locate scans), same tracks; identical results required.
+    # The mixed-precision navigator (which selects the ABBox kernels: they
+    # preselect daughters in FP32), same tracks; identical results required.
     ref_ns, ref_hash = out.nsteps.clone(), out.hash.clone()
     ref_fin = [a.clone() for a in out.final]
     mout = N.TraceResult(n, dev)
@@ -929,7 +929,7 @@ def nav_bench(args, dev, stream, with_cpu):
     mixed_ms = float(np.mean([a.elapsed_time(b) for a, b in ev]))
     same = bool(torch.equal(mout.nsteps, ref_ns) and torch.equal(mout.hash, ref_hash)
                 and all(torch.equal(a, b) for a, b in zip(mout.final, ref_fin)))
-    res["mixed"] = {"kernel": "TraceKernel<mixed> (FP32 daughter and locate filters)", "avg_launch_ms": round(mixed_ms, 3),
+    res["mixed"] = {"kernel": "TraceKernel (the ABBox navigator's)", "avg_launch_ms": round(mixed_ms, 3),
                     "value": round(total_steps / (mixed_ms * 1e-3) / 1e9, 4), "unit": "G steps/s",
                     "identical_to_fp64": same, "speedup_vs_fused_fp64": round(fused_ms / mixed_ms, 3)}
     # Plain form: one launch per step from the host.
@@ -1021,7 +1021,7 @@ def serve_bench(args, dev):
            "saturation_basket_rate_per_basket_form": round(base_rate, 1),
            "saturation_basket_rate_batched_form": round(batched_rate, 1),
            "fixed_rates": rates, "dtype": "f64",
-           "forms": "batched_mixed: requests merged into shared launches, mixed-precision ABBox navigator; batched: "
+           "forms": "batched_mixed: requests merged into shared launches, mixed-precision ABBox navigator (the same kernels); batched: "
                     "the same with the FP64 navigator; per_basket: one launch per request, one at a time, FP64"}
     for srv in servers.values():
         srv.destroy()

@@ -1,6 +1,5 @@
 // FP32 distance bounds: the single-precision filter of the mixed-precision
-// forms (shape queries with float inputs, and the navigator's daughter
-// walk).
+// shape queries (float inputs).
 //
 // For a placed volume and a point p in its mother frame, Bound32 computes in
 // FP32 two numbers:

@@ -2,6 +2,8 @@
 queries through the Python checks and ctypes: outputs, given outputs, optional
 arguments, lists for tuples, empty baskets, another stream, and the
 refusals."""
+import os
+
 import numpy as np
 import pytest
 
@@ -15,6 +17,9 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module")
 def world():
     Q.init(0)
+    if not os.path.exists(Q._FRONT_PATH):
+        pytest.skip("the native front is not built here")
+    assert Q._load_front(), "the native front is built and does not load"
     xf = W.random_placement(np.random.Generator(np.random.Philox(88)))
     geom, ids, _ = G.single_shape_geometry([dict(W.zoo_shapes())["Tube"]], [xf])
     yield geom, ids[0], xf

@@ -8,6 +8,7 @@ unless `out` is given.  Work is enqueued on torch's current stream.
 import ctypes
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -16,35 +17,41 @@ from . import capi
 # Output types and argument lists of the native front (csrc/py_queries.cpp).
 _U8, _I32, _F64 = 0, 1, 2
 _POINTS, _RAYS, _RAYS_NEXT, _NORMAL, _RAYS_NORMAL = range(5)
-_front = None
+_FRONT_PATH = os.path.join(capi.HERE, "lib", "_vgq.so")
+_front = None  # the front's run(), or False where it cannot be loaded
 _address = {}
 
 
 def _load_front():
-    """Loads the native front and the entry points' addresses once; raises if
-    it is not built."""
+    """Loads the native front and the entry points' addresses once.  It only
+    shortens the host's part of a call: where it was not built, or was built
+    against another torch, every query takes the Python checks below instead,
+    into the same library."""
     global _front
-    path = os.path.join(capi.HERE, "lib", "_vgq.so")
-    if not os.path.exists(path):
-        raise RuntimeError(f"{path} is missing: build it with __graft_entry__.build()")
     lib = capi.lib()
+    try:
+        spec = importlib.util.spec_from_file_location("vecgeom_amd._vgq", _FRONT_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError as e:  # missing file, missing symbol, other interpreter
+        warnings.warn(f"basket queries go without their native front: {e}", RuntimeWarning, stacklevel=4)
+        _front = False
+        return _front
     for name in ("vg_contains", "vg_inside", "vg_distance_to_in", "vg_distance_to_out", "vg_placed_distance_to_out",
                  "vg_safety_to_in", "vg_safety_to_out", "vg_unplaced_contains", "vg_normal",
                  "vg_distance_to_out_normal"):
         _address[name] = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
-    spec = importlib.util.spec_from_file_location("vecgeom_amd._vgq", path)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
     _front = module.run
     return _front
 
 
 def _native(name, family, geom, placed, p, d=None, step_max=None, out=None, code=_F64, next_node=None):
-    """The query through the native front: its output, or None where the
-    arguments are not the usual ones (the callers' own checks then say why)."""
-    run = _front or _load_front()
+    """The query through the native front: its output, or None where there is
+    no front or the arguments are not the usual ones (the callers' own checks
+    then say why)."""
+    run = _front if _front is not None else _load_front()
     handle = geom.handle
-    if handle is None:
+    if not run or handle is None:
         return None
     r = run(_address[name], family, handle.value, placed, p, d, step_max, out, code, next_node)
     if r is None:

@@ -635,6 +635,7 @@ VGA_NAV constexpr bool Abbox(int way) { return way == kWayAbbox || way == kWayAb
 // ------------------------------------------------------------ ABBox search
 constexpr float kReach = 4.f;  // growth of the searched stretch
 constexpr float kNear = 8.f;   // a step within this many first stretches is searched at once
+constexpr float kLeast = 1e-6f;  // shortest first stretch, as a share of the way to its begin
 
 struct Ray {
   float p[3];
@@ -679,11 +680,27 @@ VGA_NAV Ray MakeRay(V3 lp, V3 ld) {
   return r;
 }
 
+// Where the next stretch to search ends, given its begin T0, the end T of
+// the one searched before (0: none) and the step known: at the step where
+// that is near, else kReach times as far as before, and never beyond T1.
+//
+// The search ends: floats at T0 lie less than 1.2e-7 T0 apart, so a first
+// stretch of kLeast T0 or more ends beyond T0, every later one is longer than
+// the one before it, and T reaches T1 or the step (or infinity, which is T1).
+VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
+  if (!way.index) return 0.f;
+  const float first = way.index->first, least = kLeast * T0;
+  const float far = T0 + (T > 0.f ? kReach * (T - T0) : first > least ? first : least);
+  const double to = step * (1. + 1e-6) + 1e-6;  // not below step as a float
+  const float end = to <= (double)(T0 + kNear * first) || to <= (double)far ? (float)to : far;
+  return end < T1 ? end : T1;
+}
+
 // The candidate walk of ABBoxNavigator::FindNextBoundaryAndStep
 // (ABBoxNavigator.h:296-333) over daughters [db, de).  On entry `step`
 // holds the mother's DistanceToOut (kInfinity if negative).  Returns 1 if
-// the exact sorted-order walk was needed.  ExactOnly skips the order-free
-// walk (used by the host-side checks of the exact walk).
+// the exact sorted-order walk was needed.  kWayAbboxSorted skips the
+// order-free walk (used by the host-side checks of the exact walk).
 //
 // The walk searches the ray in growing stretches from its start: the
 // daughters whose extents the stretch can meet, less those seen already, in
@@ -698,18 +715,7 @@ VGA_NAV Ray MakeRay(V3 lp, V3 ld) {
 // the hits in ascending (entry distance, daughter index) order, the order of
 // a stable sort of the hit list, by repeated selection of the next one.  Both
 // orders share the code that evaluates a daughter.
-// Where the next stretch to search ends, given its begin T0, the end T of
-// the one searched before (0: none) and the step known: at the step where
-// that is near, else kReach times as far as before, and never beyond T1.
-VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
-  if (!way.index) return 0.f;
-  const float first = way.index->first;
-  const float far = T > 0.f ? T0 + kReach * (T - T0) : T0 + first;
-  const double to = step * (1. + 1e-6) + 1e-6;  // not below step as a float
-  const float end = to <= (double)(T0 + kNear * first) || to <= (double)far ? (float)to : far;
-  return end < T1 ? end : T1;
-}
-
+//
 // SimpleNavigator's loop over the daughters (kWaySimple, kWayBasket) is the
 // same search without the box tests: it takes the smallest DistanceToIn, of
 // equal ones the daughter with the lowest index (an index-order loop with a

@@ -166,6 +166,11 @@ void *navhost_geom_create(int n_shapes, const int *shape_type, const int *shape_
 
 void navhost_geom_destroy(void *h) { delete static_cast<HostGeom *>(h); }
 
+// Takes the daughter indexes away: every walk looks at every daughter.
+void navhost_drop_indexes(void *h) {
+  for (auto &r : static_cast<HostGeom *>(h)->g.nav) r.index = -1;
+}
+
 int navhost_geom_max_depth(void *h) { return static_cast<HostGeom *>(h)->g.max_depth; }
 
 void navhost_locate(void *hv, long n, const double *x, const double *y, const double *z, int depth, int *level,

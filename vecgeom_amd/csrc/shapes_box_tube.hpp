@@ -62,6 +62,11 @@ struct BoxS {
     if (s2 >= mt && p.z * dir.z < 0 && Abs(c1) <= b.d[0] && Abs(c2) <= b.d[1]) return next;
     return kInfinity;
   }
+  // Whether DistanceToIn gives dist under every step limit beyond dist, where
+  // it gave dist under one of them.
+  static VGA_HD bool LimitFree(const P &b, V3 p, double dist) {
+    return Abs(p.x) - b.d[0] <= dist && Abs(p.y) - b.d[1] <= dist && Abs(p.z) - b.d[2] <= dist;
+  }
   static VGA_HD double DistanceToOut(const P &b, V3 p, V3 dir, double) {
     const double ix = 1. / (dir.x + kMinimum), iy = 1. / (dir.y + kMinimum), iz = 1. / (dir.z + kMinimum);
     const double dx = (dir.x < 0 ? (-b.d[0] - p.x) : (b.d[0] - p.x)) * ix;

@@ -242,6 +242,12 @@ struct ParaS {
     const BoxP b{{q.d[0], q.d[1], q.d[2]}};
     return BoxS::DistanceToIn(b, Shear(q, p), Shear(q, d), stepMax);
   }
+  // The sheared excesses are no distances: they can exceed the distance to
+  // the shape, and a limit between the two hides a shape that is nearer.
+  static VGA_HD bool LimitFree(const P &q, V3 p, double dist) {
+    const BoxP b{{q.d[0], q.d[1], q.d[2]}};
+    return BoxS::LimitFree(b, Shear(q, p), dist);
+  }
   static VGA_HD double DistanceToOut(const P &q, V3 p, V3 dir, double) {
     double distance = kInfinity;
     bool inDir = dir.z > 0;

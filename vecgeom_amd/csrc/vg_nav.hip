@@ -39,13 +39,13 @@
 //    with a negative entry distance contains the point, (b) every
 //    DistanceToIn result is >= 0 and >= its box entry distance (boxes bound
 //    their shapes, so a box skipped by the sorted walk cannot hold a nearer
-//    surface), and (c) the smallest distance is reached by one daughter
-//    only.  The lane checks (a)-(c) and otherwise redoes the step in exact
-//    sorted order by repeated selection of the next (distance, index) pair.
-//    Every device shape's DistanceToIn returns the same value for any
-//    stepMax larger than that value (Box and Parallelepiped use stepMax
-//    only to return kInfinity early; the others ignore it), which is what
-//    makes the larger stepMax of the order-free walk safe.
+//    surface), (c) the smallest distance is reached by one daughter only,
+//    and (d) that distance is the same under every larger stepMax.  The lane
+//    checks (a)-(d) and otherwise redoes the step in exact sorted order by
+//    repeated selection of the next (distance, index) pair.  (d) can fail for
+//    the Parallelepiped (and for a Box by the rounding of a corner): its
+//    early exit compares a sheared safety, which is no lower bound of the
+//    distance, with stepMax.
 #include <hip/hip_runtime.h>
 
 #include <cstring>

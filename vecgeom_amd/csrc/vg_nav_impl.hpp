@@ -696,6 +696,30 @@ VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
   return end < T1 ? end : T1;
 }
 
+// Whether the best daughter's distance can depend on the step limit.  Only
+// the Box and the Parallelepiped look at the limit in a way that can change
+// an answer below it (the Polyhedron returns the limit in the place of a
+// larger distance).  A Box's excesses exceed its distance only for a point
+// inside it, or by rounding at nearly equal distances: the ABBox walk orders
+// the first case and gives every daughter the first step as limit in the
+// second; the Simple ones ask.
+enum Limited : int { kLimitFree, kLimited, kSheared };  // kSheared: a Parallelepiped, looked at in the end
+template <uint32_t M, int Way>
+VGA_NAV int LimitedBy(const NavDev &g, int id, const Head &h, V3 p, double dist) {
+  if constexpr (!Abbox(Way))
+    if ((h.code & kNavFormMask) == kFormBox)
+      return BoxS::LimitFree(BoxP{{h.s[0], h.s[1], h.s[2]}}, p, dist) ? kLimitFree : kLimited;
+  if constexpr ((M >> VG_PARALLELEPIPED) & 1u)
+    if ((h.code & kNavFormMask) == kFormGeneral && g.Nav(id).type == VG_PARALLELEPIPED) return kSheared;
+  return kLimitFree;
+}
+// The Parallelepiped `id` at distance dist from lp of its mother's frame.
+VGA_NAV bool ShearedLimitFree(const NavDev &g, int id, V3 lp, double dist) {
+  const NavRec &r = g.Nav(id);
+  const V3 p = XfPointRt(LoadXf(g, id, r.code), KindOf(r.code), lp);
+  return ParaS::LimitFree(ParamView<ParaS>::Get(g.params + r.param_off), p, dist);
+}
+
 // The candidate walk of ABBoxNavigator::FindNextBoundaryAndStep
 // (ABBoxNavigator.h:296-333) over daughters [db, de).  On entry `step`
 // holds the mother's DistanceToOut (kInfinity if negative).  Returns 1 if
@@ -707,9 +731,13 @@ VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
 // index order; it ends with the first stretch that reaches the best step
 // found.  Every daughter left lies beyond that step: it cannot contain the
 // start, and its DistanceToIn exceeds the step, so it can neither win nor
-// tie.  The order does not matter to the outcome.  That argument needs the
-// shapes' distances to be distances, which takes a unit direction; any other
-// direction takes every daughter at once.
+// tie.  That argument needs the shapes' distances to be distances, which
+// takes a unit direction; any other direction takes every daughter at once.
+//
+// Every daughter is given the first step as limit, not the running one: a
+// limit only takes away answers, and the winner under the first limit is the
+// winner in any order, if its distance does not depend on the limit
+// (Limited).
 //
 // Where the outcome does depend on the order the walk starts again and takes
 // the hits in ascending (entry distance, daughter index) order, the order of
@@ -719,7 +747,8 @@ VGA_NAV float Reach(const Meet &way, float T0, float T1, float T, double step) {
 // SimpleNavigator's loop over the daughters (kWaySimple, kWayBasket) is the
 // same search without the box tests: it takes the smallest DistanceToIn, of
 // equal ones the daughter with the lowest index (an index-order loop with a
-// strict comparison).
+// strict comparison); where the winner depends on the limit, it walks again
+// over every daughter in index order with the running step as limit.
 template <uint32_t M, int Way>
 VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &step, int &next) {
   const int db = C.dbegin;
@@ -744,6 +773,7 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
   float behind = 0.f;
   bool sorted = Way == kWayAbboxSorted;
   int ties = 0;
+  int limited = kLimitFree;  // of the best step
   float lastb = -kInfF;
   int lastk = -1;
   next = -1;
@@ -761,10 +791,20 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
           }
         } else {
           if (!way.index || T >= T1 || step <= (double)T) {
-            if (!Abbox(Way) || ties <= 1) return 0;
-            sorted = true;
+            if constexpr ((M >> VG_PARALLELEPIPED) & 1u)
+              if (limited == kSheared && ShearedLimitFree(g, g.Daughter(db + next), lp, step)) limited = kLimitFree;
+            if ((!Abbox(Way) || ties <= 1) && limited == kLimitFree) return 0;
             step = step0;
             next = -1;
+            if constexpr (Abbox(Way)) {
+              sorted = true;
+            } else {
+              limited = kLimitFree;
+              way.index = nullptr;
+              behind = 0.f;
+              w = 0;
+              m = way.Mask(g, 0);
+            }
             continue;
           }
           behind = T;
@@ -810,15 +850,15 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
       next = k;
       return 1;
     }
-    // SimpleNavigator's step limit is the running step; with the index, whose
-    // order is another, the first one (no answer below the step depends on
-    // it for a unit direction).
+    // The limit: the running step where the daughters come in the navigator's
+    // own order, else the first one.
     const double sm = (Abbox(Way) ? sorted : !way.index) ? step : step0;
     const double dd = NDistIn<M>(g, cand, h, tp, XfDirRt(x, KindOf(h.code), ld), sm);
     if (!Abbox(Way)) {
       if ((dd < step || (dd == step && k < next)) && !(Way == kWaySimple && __builtin_isinf(dd))) {
         step = dd;
         next = k;
+        if (way.index) limited = LimitedBy<M, Way>(g, cand, h, tp, dd);
       }
     } else if (sorted) {
       if (dd < step) {
@@ -833,6 +873,7 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
       step = dd;
       next = k;
       ties = 1;
+      limited = LimitedBy<M, Way>(g, cand, h, tp, dd);
     } else if (dd == step) {
       ++ties;
     }

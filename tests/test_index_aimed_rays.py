@@ -83,3 +83,37 @@ def test_aimed_rays(oracle, hostnav, names, n, half):
     for kind in (0, 1):
         for x, y in zip(want.trace(p, d, kind=kind, nthreads=8), H.trace(p, d, kind=kind, nthreads=8)):
             assert same(x, y).all(), (names, kind)
+
+
+@pytest.mark.parametrize("names,n", [("exact", 30), ("all", 80), ("grazed", 70)])
+@pytest.mark.parametrize("how", ["float", 1.0 + 4.9e-7, 1.0 - 4.9e-7, 1.0 + 1e-3, 1.0 + 1e-9])
+def test_directions_near_unit_length(hostnav, names, n, how):
+    """Directions that were stored as float, or a little longer or shorter
+    than a unit vector, up to the length where the index is left aside and
+    beyond: the index changes nothing.  "grazed": rays along an axis that pass
+    round shapes of half-width 50 mm at a distance to which such a direction
+    shifts their tangents (from 10^5 mm, 10^10 * 1e-6 / 100 = 100 mm)."""
+    half = 100000.0 if names == "grazed" else 2000.0
+    round_ones = ["Orb", "Tube", "Cone", "Paraboloid", "Torus", "Polycone"]
+    flat, centres = world_of(round_ones if names == "grazed" else SETS[names], n, half, W.SEED_BASE + 460)
+    H, want = po.Nav(hostnav, flat), po.Nav(hostnav, flat)
+    hostnav.lib.navhost_drop_indexes(ctypes.c_void_p(want.h))
+    p, d = aimed(60000, half, centres, 23)
+    if names == "grazed":  # along an axis, so that one coordinate decides
+        rng = np.random.Generator(np.random.Philox(29))
+        n = p.shape[1]
+        axis, sign = rng.integers(0, 3, n), rng.choice((-1.0, 1.0), n)
+        c = centres[:, rng.integers(0, centres.shape[1], n)]
+        d = np.zeros((3, n))
+        d[axis, np.arange(n)] = sign
+        p = c.copy()
+        p[axis, np.arange(n)] = -sign * 0.99 * half
+        p[(axis + 1) % 3, np.arange(n)] += (50.0 + rng.uniform(-1.0, 40.0, n)) * rng.choice((-1.0, 1.0), n)
+    d = d.astype(np.float32).astype(np.float64) if how == "float" else d * how
+    level, path = want.locate(p, nthreads=8)
+    for kind in KINDS[:2]:
+        for x, y in zip(want.step(p, d, level, path, kind=kind, nthreads=8),
+                        H.step(p, d, level, path, kind=kind, nthreads=8)):
+            assert same(x, y).all(), (kind, int((~same(x, y)).sum()))
+        for x, y in zip(want.trace(p, d, kind=kind, nthreads=8), H.trace(p, d, kind=kind, nthreads=8)):
+            assert same(x, y).all(), (kind, int((~same(x, y)).sum()))

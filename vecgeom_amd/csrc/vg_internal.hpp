@@ -42,6 +42,8 @@ constexpr int kNavTurns = 1 << 6;      // r is read: a rotation about z, r[0], r
 constexpr int kNavMatrix = 1 << 7;     // the placement is read from the PlacedRec
 constexpr int kNavAxesShift = 8;       // coordinates of the daughter index: count (2 bits),
 constexpr int kNavCoordShift = 10;     // then 2 bits each
+constexpr int kNavWalks = 1 << 16;     // the ABBox daughter search uses the index (locate and safety always do)
+constexpr int kNavWalksSimple = 1 << 17;  // the Simple navigators' does
 struct alignas(128) NavRec {
   int32_t code;
   int32_t index;   // daughter index of its logical volume (-1: none)

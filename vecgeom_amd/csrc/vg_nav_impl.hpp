@@ -684,6 +684,31 @@ VGA_NAV float IntersectBox(const float *b, const Ray &r) {
   return tmin;
 }
 
+// Which of n boxes (64 at most) the ray hits (IntersectBox below infinity), as
+// a bit mask: the full walk's box tests, without branches so that the loads of
+// several boxes are in flight at once (traces of 262,144 tracks in a world of 6
+// boxes 191 -> 119 us, of nine shapes 421 -> 292).
+VGA_NAV uint64_t Hits(const NavDev &g, int slot, int n, const Ray &r) {
+  uint64_t hit = 0;
+#pragma unroll 4
+  for (int k = 0; k < n; ++k) {
+    const float *b = g.SlotBox(slot + k);
+    float tmin = -kInfF, tmax = kInfF;
+    bool miss = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float lo = ((r.sign[a] ? b[3 + a] : b[a]) - r.p[a]) * r.inv[a];
+      const float hi = ((r.sign[a] ? b[a] : b[3 + a]) - r.p[a]) * r.inv[a];
+      if (a > 0) miss |= (tmin > hi) | (lo > tmax);
+      tmin = a > 0 && !(tmin < lo) ? tmin : lo;
+      tmax = a > 0 && !(hi < tmax) ? tmax : hi;
+    }
+    miss |= !((tmin < kInfF) & (tmax > 0.f));
+    hit |= (uint64_t)!miss << k;
+  }
+  return hit;
+}
+
 VGA_NAV Ray MakeRay(V3 lp, V3 ld) {
   Ray r;
   r.inv[0] = 1.f / (float)ld.x;
@@ -776,7 +801,13 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
   const double step0 = step;
   const double off = Abs(ld.Mag2() - 1.);
   const float slack = Slack(off);
-  Meet way(g, C.code, C.index, C.nd, Finite(lp) && off < kNearUnit);
+  Meet way(g, C.code, C.index, C.nd, (C.code & (Abbox(Way) ? kNavWalks : kNavWalksSimple)) && Finite(lp) && off < kNearUnit);
+  // Word w of the daughters to look at.
+  auto word = [&](int w) {
+    if constexpr (Abbox(Way))
+      if (!way.index) return Hits(g, db + 64 * w, C.nd - 64 * w < 64 ? C.nd - 64 * w : 64, ray);
+    return way.Mask(g, w);
+  };
   const F3 fp{ray.p[0], ray.p[1], ray.p[2]}, fd{(float)ld.x, (float)ld.y, (float)ld.z};
   // The stretch [T0, T] of the ray is searched next; beyond T1 it meets no
   // daughter.
@@ -790,7 +821,7 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
   } else {
     T = Reach(way, T0, T1, 0.f, step);
     way.Stretch(fp, fd, T0, T, slack);
-    seen = m = way.Mask(g, 0);
+    seen = m = word(0);
   }
   float behind = 0.f;
   bool sorted = Way == kWayAbboxSorted;
@@ -805,7 +836,7 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
     if (!sorted) {
       if (!m) {
         if (++w < way.words) {
-          m = way.Mask(g, w);
+          m = word(w);
           if (behind > 0.f) {
             Meet before = way;
             before.Stretch(fp, fd, T0, behind, slack);

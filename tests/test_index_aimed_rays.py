@@ -117,3 +117,32 @@ def test_directions_near_unit_length(hostnav, names, n, how):
             assert same(x, y).all(), (kind, int((~same(x, y)).sum()))
         for x, y in zip(want.trace(p, d, kind=kind, nthreads=8), H.trace(p, d, kind=kind, nthreads=8)):
             assert same(x, y).all(), (kind, int((~same(x, y)).sum()))
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
+def test_safety_among_safe_daughters(oracle, hostnav, n, scale):
+    """Orbs and boxes turned about z, from the number of daughters where the
+    safety takes the index on: points near them, in them, and beyond."""
+    rng = np.random.Generator(np.random.Philox(W.SEED_BASE + 470 + n))
+    gm = G.GeoManager()
+    half = 400.0 * scale
+    world = G.LogicalVolume("world", G.UnplacedBox(half, half, half), gm)
+    lv = [G.LogicalVolume("box", G.UnplacedBox(10 * scale, 30 * scale, 5 * scale), gm),
+          G.LogicalVolume("orb", G.UnplacedOrb(12 * scale), gm)]
+    for i in range(n):
+        f = rng.uniform(0, 2 * math.pi)
+        c, s = math.cos(f), math.sin(f)
+        at = rng.uniform(-0.6, 0.6, 3) * half
+        turn = [c, -s, 0.0, s, c, 0.0, 0.0, 0.0, 1.0] if i % 2 == 0 else []
+        world.PlaceDaughter(f"d{i}", lv[i % 2], G.Transformation3D(*at, *turn))
+    gm.SetWorld(world.Place("world"))
+    flat = gm.CloseGeometry()
+    O, H = po.Nav(oracle, flat), po.Nav(hostnav, flat)
+    p = rng.uniform(-1.0, 1.0, (3, 8000)) * half
+    p[:, :1000] *= 1e3  # outside the world
+    p[0, 1000:1200] = half * (1 - rng.uniform(0, 1e-9, 200))  # at its wall
+    level = np.ones(p.shape[1], np.int32)
+    path = np.full((O.depth, p.shape[1]), -1, np.int32)
+    path[0] = flat.world
+    assert same(O.safety(p, level, path, nthreads=8), H.safety(p, level, path, nthreads=8)).all()

@@ -16,6 +16,11 @@ constexpr int kSamples = 256;  // points at which coordinates are compared
 // First stretch of a ray to search, as a share of the diagonal of the
 // daughters' extent.
 constexpr double kFirst = 1. / 512;
+// First distance to search for a safety, as a share of the diagonal over the
+// cube root of the number of daughters (the pitch of a cubic grid is 0.58):
+// 262,144 points scattered in the nested geometry 43 us from 1/512 of the
+// diagonal, 38 with 0.12, 49 with 0.2, 70 with 0.35.
+constexpr double kNearShare = 0.12;
 
 // Local extent along z and from the z axis of a shape that turns about z
 // (rlo is 0 where the hollow's depth is not bounded simply).
@@ -160,8 +165,9 @@ DaughterIndex BuildDaughterIndex(const std::vector<DaughterExtent> &d, std::vect
   diag = std::sqrt(diag);
   const int n = Slices(nd);
   ix.first = (float)std::max(diag * kFirst, 1e-6);
-  ix.safe = 1;
-  for (const auto &e : d) ix.safe &= e.safe ? 1 : 0;
+  ix.near = (float)std::max(diag * kNearShare / std::cbrt((double)nd), 1e-6);
+  axes->safe = true;
+  for (const auto &e : d) axes->safe &= e.safe;
   for (int c = 0; c < 3; ++c) {
     const double pad = 1e-3 + 1e-6 * size;
     ix.lo[c] = (float)(lo[c] - pad);

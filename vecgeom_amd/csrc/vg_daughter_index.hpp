@@ -36,16 +36,18 @@ struct DaughterAxis {
 
 struct DaughterIndex {
   float first;         // first stretch of a ray to search (mm)
-  int32_t safe;        // 1: see DaughterExtent::safe, for every daughter
+  float near;          // first distance around a point to search for its safety (mm)
   float lo[3], hi[3];  // box of all daughters' extents
   DaughterAxis axis[kIndexAxes];
 };
 static_assert(sizeof(DaughterIndex) == 80, "five 16-byte loads");
 
-// Which coordinates an index looks up: the first `count` entries of coord.
+// Which coordinates an index looks up: the first `count` entries of coord; and
+// whether every daughter is safe (DaughterExtent::safe).
 struct IndexAxes {
   int count = 0;
   int coord[kIndexAxes] = {};
+  bool safe = false;
 };
 
 // One daughter's extent in its mother's frame: x, y, z and rho.

@@ -188,6 +188,8 @@ struct WalkMin {
   int abbox, simple;
 };
 constexpr WalkMin kWalkWorld = {20, 9}, kWalkWorldGeneral = {32, 20}, kWalkBelow = {8, 8}, kWalkBelowGeneral = {12, 12};
+// The safety takes the index from kSafeMin daughters on (figures at GetSafety).
+constexpr int kSafeMin = 32;
 constexpr size_t kIndexMaxWords = size_t(1) << 25;  // 256 MiB
 
 void BuildIndexes(vg_geometry *g) {
@@ -218,7 +220,10 @@ void BuildIndexes(vg_geometry *g) {
     const WalkMin min = top ? (basic ? kWalkWorld : kWalkWorldGeneral) : (basic ? kWalkBelow : kWalkBelowGeneral);
     if (de - db >= min.abbox) axes_code[l] |= kNavWalks;
     if (de - db >= min.simple) axes_code[l] |= kNavWalksSimple;
+    if (axes.safe && de - db >= kSafeMin) axes_code[l] |= kNavSafe;
   }
+  for (int l = 0; l < nl; ++l)
+    g->safety_scans |= g->logical_dbegin[l + 1] - g->logical_dbegin[l] >= kIndexMinDaughters && !(axes_code[l] & kNavSafe);
   g->nav.resize(g->placed.size());
   for (size_t p = 0; p < g->placed.size(); ++p) {
     const PlacedRec &r = g->placed[p];

@@ -42,8 +42,9 @@ constexpr int kNavTurns = 1 << 6;      // r is read: a rotation about z, r[0], r
 constexpr int kNavMatrix = 1 << 7;     // the placement is read from the PlacedRec
 constexpr int kNavAxesShift = 8;       // coordinates of the daughter index: count (2 bits),
 constexpr int kNavCoordShift = 10;     // then 2 bits each
-constexpr int kNavWalks = 1 << 16;     // the ABBox daughter search uses the index (locate and safety always do)
+constexpr int kNavWalks = 1 << 16;     // the ABBox daughter search uses the index (locate always does)
 constexpr int kNavWalksSimple = 1 << 17;  // the Simple navigators' does
+constexpr int kNavSafe = 1 << 18;      // the safety does
 struct alignas(128) NavRec {
   int32_t code;
   int32_t index;   // daughter index of its logical volume (-1: none)
@@ -102,6 +103,7 @@ struct vg_geometry {
   double *d_scalar = nullptr;  // device staging of vg_scalar_query (16 doubles)
   std::mutex scalar_mutex;     // one vg_scalar_query at a time per geometry
   int32_t nav_bad_type = 0;  // first shape type in the tree without device kernels (0: none)
+  bool safety_scans = false; // some volume's safety looks at every daughter
   uint32_t type_mask = 0;    // bit t set: some placed volume has shape type t (bit 0: a Tube with a phi section)
 };
 

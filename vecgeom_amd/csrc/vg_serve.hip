@@ -143,8 +143,16 @@ __global__ __launch_bounds__(kServeBlock) void ServeReadKernel(const Arena a, co
 // (level 0) stays where it is with step 0.  Tiles of kServeBlock lanes
 // ((kServeBlock / 64) << shift tracks, LanesShift) are numbered across
 // segments; each block finds its segment by binary search.
+//
+// Occupancy floors as those of the trace kernel: over all shapes the compiler
+// would take 330 registers and run one wave per SIMD, and a basket's first step
+// in the nine shapes' geometry took longer than before the daughter index
+// (16,384 tracks 72 -> 85 us, with two waves 62; 262,144 tracks 256 -> 206 and
+// 176); over the basic shapes three waves cost a few spills at depth 8 and 16.
+constexpr int ServeWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 3 : 2; }
+
 template <int D, uint32_t M, int Way>
-__global__ __launch_bounds__(kServeBlock) void ServeStepKernel(const NavDev g, const Arena a,
+__global__ __launch_bounds__(kServeBlock) __attribute__((amdgpu_waves_per_eu(ServeWaves(M)))) void ServeStepKernel(const NavDev g, const Arena a,
                                                                const Seg *__restrict__ segs, int nseg, uint64_t ntiles,
                                                                double pstep, int shift) {
   const uint64_t tile = blockIdx.x;

@@ -78,18 +78,20 @@ void Step(const HostGeom *h, long n, const double *x, const double *y, const dou
       DPath<D> o;
       Load(level_in, path_in, n, i, o);
       double step = 0;
+      NavDev dev = h->dev;
+      dev.walks = WalkBit(kind != VG_NAV_SIMPLE && kind != VG_NAV_SIMPLE_BASKET, n < (long)kBigStep ? kWalkStep : kWalkBigStep);
       const V3 q{x[i], y[i], z[i]}, v{dx[i], dy[i], dz[i]};
       if (kind == VG_NAV_SIMPLE_BASKET) {
         DPath<D> c0;
         Load(level_in, path_in, n, 0, c0);
         if (o.level > 0 && c0.level > 0)
-          FindNextBoundaryAndStep<D, kAllShapes, kWayBasket>(h->dev, q, v, o, pstep, step, c0.Top());
+          FindNextBoundaryAndStep<D, kAllShapes, kWayBasket>(dev, q, v, o, pstep, step, c0.Top());
       } else if (o.level > 0 && kind == kExactOnlyKind) {
-        FindNextBoundaryAndStep<D, kAllShapes, kWayAbboxSorted>(h->dev, q, v, o, pstep, step, o.Top());
+        FindNextBoundaryAndStep<D, kAllShapes, kWayAbboxSorted>(dev, q, v, o, pstep, step, o.Top());
       } else if (o.level > 0 && kind == VG_NAV_SIMPLE) {
-        FindNextBoundaryAndStep<D, kAllShapes, kWaySimple>(h->dev, q, v, o, pstep, step, o.Top());
+        FindNextBoundaryAndStep<D, kAllShapes, kWaySimple>(dev, q, v, o, pstep, step, o.Top());
       } else if (o.level > 0) {
-        FindNextBoundaryAndStep<D, kAllShapes, kWayAbbox>(h->dev, q, v, o, pstep, step, o.Top());
+        FindNextBoundaryAndStep<D, kAllShapes, kWayAbbox>(dev, q, v, o, pstep, step, o.Top());
       }
       Store(o, depth, n, i, level_out, path_out);
       boundary_out[i] = (unsigned char)o.boundary;
@@ -121,11 +123,13 @@ void Trace(const HostGeom *h, long n, const double *x, const double *y, const do
       uint64_t hh;
       int nexact;
       const V3 dd{dx[i], dy[i], dz[i]};
+      NavDev dev = h->dev;
+      dev.walks = WalkBit(kind != VG_NAV_SIMPLE, kWalkTrace);
       nsteps[i] = kind == kExactOnlyKind
-                      ? TraceOne<D, kAllShapes, kWayAbboxSorted>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact)
+                      ? TraceOne<D, kAllShapes, kWayAbboxSorted>(dev, p, dd, pstep, max_steps, dist, hh, nexact)
                   : kind == VG_NAV_SIMPLE
-                      ? TraceOne<D, kAllShapes, kWaySimple>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact)
-                      : TraceOne<D, kAllShapes, kWayAbbox>(h->dev, p, dd, pstep, max_steps, dist, hh, nexact);
+                      ? TraceOne<D, kAllShapes, kWaySimple>(dev, p, dd, pstep, max_steps, dist, hh, nexact)
+                      : TraceOne<D, kAllShapes, kWayAbbox>(dev, p, dd, pstep, max_steps, dist, hh, nexact);
       fx[i] = p.x;
       fy[i] = p.y;
       fz[i] = p.z;
@@ -161,6 +165,7 @@ void *navhost_geom_create(int n_shapes, const int *shape_type, const int *shape_
   h->dev.n_daughters = (int32_t)h->g.daughters.size();
   h->dev.n_index = (int32_t)h->g.dindex.size();
   h->dev.n_masks = (int32_t)h->g.dmasks.size();
+  h->dev.walks = 0;
   return h;
 }
 

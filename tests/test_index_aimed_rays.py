@@ -146,3 +146,32 @@ def test_safety_among_safe_daughters(oracle, hostnav, n, scale):
     path = np.full((O.depth, p.shape[1]), -1, np.int32)
     path[0] = flat.world
     assert same(O.safety(p, level, path, nthreads=8), H.safety(p, level, path, nthreads=8)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("names,n", [("planar", 4), ("planar", 33), ("exact", 20), ("exact", 101), ("boxes", 65)])
+def test_steps_on_the_device(oracle, names, n):
+    """Launches on both sides of the sizes and numbers of daughters where a
+    step takes the index, the loop, and full waves."""
+    import torch
+
+    from vecgeom_amd import nav as N
+    from vecgeom_amd import queries as Q
+    Q.init(0)
+    flat, centres = world_of(["Box"] if names == "boxes" else SETS[names], n, 1200.0, W.SEED_BASE + 480 + n)
+    O, geom = po.Nav(oracle, flat), G.DeviceGeometry(flat)
+    host = lambda a: a.cpu().numpy()
+    for tracks in (200, 32767, 32768):
+        p, d = aimed(tracks, 1200.0, centres, 31)
+        t = lambda a: tuple(torch.from_numpy(np.ascontiguousarray(a[i])).to("cuda:0") for i in range(3))
+        tp, td = t(p), t(d)
+        level, path = O.locate(p, nthreads=8)
+        cur = N.locate_points(geom, tp)
+        assert (host(cur.level) == level).all() and (host(cur.path) == path).all()
+        assert same(host(N.get_safety(geom, tp, cur)), O.safety(p, level, path, nthreads=8)).all()
+        for kind in KINDS:
+            new, step = N.find_next_boundary_and_step(geom, tp, td, cur, navigator=kind)
+            want = O.step(p, d, level, path, kind=kind, nthreads=8)
+            for x, y in zip(want, (new.level, new.path, new.boundary, step)):
+                assert same(x, host(y)).all(), (tracks, kind)
+    geom.free()

@@ -183,11 +183,44 @@ NavRec MakeNavRec(const PlacedRec &r, const double *blk) {
 // 1264 and 1409, 32 1381 and 1246.  In volumes below the world the lanes are in
 // different ones and the loop gains less: the nested geometry's 8 Trds in a
 // box as a loop 4.85 ms, with the index 4.5.
+//
+// In single-step kernels the lanes of a wave stay in step and the loop holds
+// out longer, most of all where waves are full (kBigStep).  262,144 tracks,
+// loop and index: ABBox 40 boxes 48 and 96 us, 96 147 and 216, 96 daughters with
+// phi tubes 319 and 327, of all shapes 989 and 1084; Simple 40 with phi tubes 158
+// and 182, 96 353 and 427, of all shapes 773 and 1294.  1,000 tracks: ABBox 64
+// boxes 37 and 28, 32 26 and 21, 24 21 and 23; Simple 24 boxes 54 and 30, 96 of
+// all shapes 260 and 250.
 constexpr int kIndexMinDaughters = 3;
 struct WalkMin {
-  int abbox, simple;
+  int abbox[3], simple[3];  // by WalkKernel
 };
-constexpr WalkMin kWalkWorld = {20, 9}, kWalkWorldGeneral = {32, 20}, kWalkBelow = {8, 8}, kWalkBelowGeneral = {12, 12};
+constexpr WalkMin kWalkWorld = {{20, 64, 100}, {9, 32, 100}}, kWalkWorldGeneral = {{32, 100, 100}, {20, 128, 128}};
+constexpr WalkMin kWalkBelow = {{8, 8, 8}, {8, 8, 8}}, kWalkBelowGeneral = {{12, 12, 12}, {12, 12, 12}};
+// Where boxes lie in one another (the nested geometry's 64 coaxial shells) box
+// tests sort out little and the loop evaluates most daughters: the minima of
+// kWalkBelow hold in the world, too.  One step of 65,536 vertex tracks there as
+// a loop 140 us, with the index 15.
+constexpr double kCrowded = 2;
+
+// The mean number of daughters whose box holds the centre of a daughter's box.
+double Crowd(const vg_geometry *g, int db, int de) {
+  long in = 0;
+  for (int k = db; k < de; ++k) {
+    const double *b = g->aabb.data() + 6 * (size_t)g->daughters[k];
+    for (int j = db; j < de; ++j) {
+      const double *o = g->aabb.data() + 6 * (size_t)g->daughters[j];
+      bool inside = true;
+      for (int a = 0; a < 3; ++a) {
+        const double c = 0.5 * (b[a] + b[3 + a]);
+        inside &= c >= o[a] && c <= o[3 + a];
+      }
+      in += inside;
+    }
+  }
+  return (double)in / (de - db);
+}
+
 // The safety takes the index from kSafeMin daughters on (figures at GetSafety).
 constexpr int kSafeMin = 32;
 constexpr size_t kIndexMaxWords = size_t(1) << 25;  // 256 MiB
@@ -216,10 +249,13 @@ void BuildIndexes(vg_geometry *g) {
     g->dindex.push_back(BuildDaughterIndex(ext, g->dmasks, &axes));
     axes_code[l] = axes.count << kNavAxesShift;
     for (int a = 0; a < axes.count; ++a) axes_code[l] |= axes.coord[a] << (kNavCoordShift + 2 * a);
-    const bool top = l == g->placed[g->world].logical;
-    const WalkMin min = top ? (basic ? kWalkWorld : kWalkWorldGeneral) : (basic ? kWalkBelow : kWalkBelowGeneral);
-    if (de - db >= min.abbox) axes_code[l] |= kNavWalks;
-    if (de - db >= min.simple) axes_code[l] |= kNavWalksSimple;
+    // (From 128 daughters on every kernel takes the index.)
+    const bool spread = l == g->placed[g->world].logical && de - db < 128 && Crowd(g, db, de) < kCrowded;
+    const WalkMin min = spread ? (basic ? kWalkWorld : kWalkWorldGeneral) : (basic ? kWalkBelow : kWalkBelowGeneral);
+    for (const WalkKernel k : {kWalkTrace, kWalkStep, kWalkBigStep}) {
+      if (de - db >= min.abbox[k]) axes_code[l] |= WalkBit(true, k);
+      if (de - db >= min.simple[k]) axes_code[l] |= WalkBit(false, k);
+    }
     if (axes.safe && de - db >= kSafeMin) axes_code[l] |= kNavSafe;
   }
   for (int l = 0; l < nl; ++l)

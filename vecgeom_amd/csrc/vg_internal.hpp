@@ -42,9 +42,11 @@ constexpr int kNavTurns = 1 << 6;      // r is read: a rotation about z, r[0], r
 constexpr int kNavMatrix = 1 << 7;     // the placement is read from the PlacedRec
 constexpr int kNavAxesShift = 8;       // coordinates of the daughter index: count (2 bits),
 constexpr int kNavCoordShift = 10;     // then 2 bits each
-constexpr int kNavWalks = 1 << 16;     // the ABBox daughter search uses the index (locate always does)
-constexpr int kNavWalksSimple = 1 << 17;  // the Simple navigators' does
-constexpr int kNavSafe = 1 << 18;      // the safety does
+constexpr int kNavSafe = 1 << 16;      // the safety uses the index (locate always does)
+// The daughter search uses the index: a bit for each kind of kernel.
+enum WalkKernel { kWalkTrace, kWalkStep, kWalkBigStep };  // a big step: kBigStep tracks or more
+constexpr uint64_t kBigStep = 32768;
+constexpr int WalkBit(bool abbox, WalkKernel k) { return 1 << (17 + (abbox ? 0 : 1) + 2 * (int)k); }
 struct alignas(128) NavRec {
   int32_t code;
   int32_t index;   // daughter index of its logical volume (-1: none)

@@ -97,9 +97,10 @@ VGA_NAV void StoreState(const vg_nav_states &s, uint64_t i, const DPath<D> &p) {
 constexpr int TraceWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 3 : 2; }
 
 // The single-step kernels: with every shape two waves as above; over the
-// basic shapes the compiler's own choice (their registers hold three or
-// more).
-constexpr int StepWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 1 : 2; }
+// basic shapes four at the price of a few spills (262,144 tracks: one ABBox
+// step of the nested geometry 27 -> 23 us, among four daughters with phi tubes
+// 36 -> 32, Simple 34 -> 29; 65,536 nested tracks 15 -> 16).
+constexpr int StepWaves(uint32_t m) { return (m & ~(kBasicShapes | kPhiTube)) == 0 ? 4 : 2; }
 
 template <int D, uint32_t M>
 __global__ __launch_bounds__(kNavBlock) void LocateKernel(const NavDev g, const double *__restrict__ x,
@@ -216,19 +217,25 @@ int NavStep(const vg_geometry *g, int kind, const double *x, const double *y, co
             const double *dy, const double *dz, const double *pstep, uint64_t n, const vg_nav_states &cur,
             const vg_nav_states &nxt, double *step, hipStream_t st) {
   if (n == 0) return VG_OK;
-  const StepArgs a{x, y, z, dx, dy, dz, pstep, step, n, LanesShift(n), 0};
+  const bool abbox = kind != VG_NAV_SIMPLE && kind != VG_NAV_SIMPLE_BASKET;
+  const int walks = WalkBit(abbox, n < kBigStep ? kWalkStep : kWalkBigStep);
+  // The Simple navigators' loop over the world's daughters evaluates all of
+  // them, all lanes the same one at a time: full waves, as for the safety.
+  const NavRec &world = g->nav[g->world];
+  const bool loop = !abbox && world.nd >= 3 && !(world.code & walks);
+  const StepArgs a{x, y, z, dx, dy, dz, pstep, step, n, loop ? 6 : LanesShift(n), 0};
   const dim3 blocks(Blocks(n, a.shift)), threads(kNavBlock);
   if (kind == VG_NAV_SIMPLE)
     WithVariant(g, [&](auto D, auto M) {
-      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g, walks), a, cur, nxt);
     });
   else if (kind == VG_NAV_SIMPLE_BASKET)
     WithVariant(g, [&](auto D, auto M) {
-      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayBasket>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayBasket>), blocks, threads, 0, st, DeviceNav(g, walks), a, cur, nxt);
     });
   else
     WithVariant(g, [&](auto D, auto M) {
-      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g), a, cur, nxt);
+      hipLaunchKernelGGL((StepKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g, walks), a, cur, nxt);
     });
   return CheckHip(hipGetLastError(), "step launch");
 }
@@ -255,11 +262,11 @@ int NavTrace(const vg_geometry *g, int kind, const double *x, const double *y, c
   const dim3 blocks(Blocks(n, a.shift)), threads(kNavBlock);
   if (kind == VG_NAV_SIMPLE)
     WithVariant(g, [&](auto D, auto M) {
-      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g), a);
+      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWaySimple>), blocks, threads, 0, st, DeviceNav(g, WalkBit(kind != VG_NAV_SIMPLE, kWalkTrace)), a);
     });
   else
     WithVariant(g, [&](auto D, auto M) {
-      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g), a);
+      hipLaunchKernelGGL((TraceKernel<D.value, M.value, kWayAbbox>), blocks, threads, 0, st, DeviceNav(g, WalkBit(kind != VG_NAV_SIMPLE, kWalkTrace)), a);
     });
   return CheckHip(hipGetLastError(), "trace launch");
 }

@@ -45,6 +45,7 @@ struct NavDev {
   int32_t n_daughters;
   int32_t n_index;
   int32_t n_masks;
+  int32_t walks;  // WalkBit of the kernel
   VGA_NAV const NavRec &Nav(int id) const {
     VGA_NAV_CHECK(id >= 0 && id < n_placed, "placed id out of range");
     return nav[id];
@@ -828,7 +829,7 @@ VGA_NAV int Candidates(const NavDev &g, const Head &C, V3 lp, V3 ld, double &ste
   const double step0 = step;
   const double off = Abs(ld.Mag2() - 1.);
   const float slack = Slack(off);
-  Meet way(g, C.code, C.index, C.nd, (C.code & (Abbox(Way) ? kNavWalks : kNavWalksSimple)) && Finite(lp) && off < kNearUnit);
+  Meet way(g, C.code, C.index, C.nd, (C.code & g.walks) && Finite(lp) && off < kNearUnit);
   // Word w of the daughters to look at.
   auto word = [&](int w) {
     if constexpr (Abbox(Way))
@@ -1169,8 +1170,8 @@ VGA_NAV uint64_t TrackOf(uint64_t thread, int shift, uint64_t n) {
   return (lane >> shift) ? n : ((thread >> 6) << shift) + lane;
 }
 
-// The navigator's view of an uploaded geometry.
-inline NavDev DeviceNav(const vg_geometry *g) {
+// The navigator's view of an uploaded geometry, for kernels of one WalkBit.
+inline NavDev DeviceNav(const vg_geometry *g, int walks = 0) {
   return NavDev{g->d_nav,
                 g->d_placed,
                 g->d_params,
@@ -1181,7 +1182,8 @@ inline NavDev DeviceNav(const vg_geometry *g) {
                 (int32_t)g->placed.size(),
                 (int32_t)g->daughters.size(),
                 (int32_t)g->dindex.size(),
-                (int32_t)g->dmasks.size()};
+                (int32_t)g->dmasks.size(),
+                walks};
 }
 
 // Calls f(D, M) with the path depth D (4, 8 or 16) that holds the geometry

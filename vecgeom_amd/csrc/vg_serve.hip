@@ -537,7 +537,7 @@ int vg_server_create(const vg_geometry *g, uint64_t hbm_budget_bytes, int32_t na
   s->g = g;
   s->navigator = navigator;
   s->pstep = pstep;
-  s->dev = DeviceNav(g);
+  s->dev = DeviceNav(g, WalkBit(navigator != VG_NAV_SIMPLE, kWalkStep));
   rc = CheckHip(hipMalloc(&s->mem, cap * SlotBytes(depth)), "hipMalloc(serve arena)");
   if (!rc) {
     char *m = static_cast<char *>(s->mem);

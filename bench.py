@@ -1066,6 +1066,26 @@ def nav_cpu_baseline(flat, p0, d0, target_s):
                       + "; one warm-up pass, median of 5 passes on one thread"}
 
 
+# What the result line keeps of a block's inner records.
+_INNER = ("value", "ms_per_step", "p50_ms", "p99_ms", "speedup_vs_fused_fp64", "identical_to_fp64", "threads")
+
+
+def summary(line):
+    """The result line: every block's own numbers and the headline numbers of
+    its inner records, without the per-kernel and per-rate tables."""
+    out = {}
+    for key, block in line.items():
+        if key in ("config", "roofline", "forms_gqps"):
+            out[key] = block
+        elif isinstance(block, dict):
+            out[key] = {k: {i: x for i, x in v.items() if i in _INNER} if isinstance(v, dict) else v
+                        for k, v in block.items() if not isinstance(v, list)}
+            out[key] = {k: v for k, v in out[key].items() if v != {}}
+        elif not isinstance(block, list):
+            out[key] = block
+    return out
+
+
 def main():
     args = parse()
     if args.gpus != 1:
@@ -1235,7 +1255,10 @@ def main():
         "normals": normals,
         "per_kernel": [{k: (round(v, 3) if isinstance(v, float) else v) for k, v in r.items()} for r in rows],
     }
-    print(json.dumps(line), flush=True)
+    # The whole record goes to stderr; the result line on stdout stays short
+    # enough for a reader that keeps the last few thousand characters.
+    log("details " + json.dumps(line))
+    print(json.dumps(summary(line)), flush=True)
 
 
 if __name__ == "__main__":

@@ -336,8 +336,8 @@ constexpr int ClassOf(int type) {
 // Items per lane of class c when the batch asks for `it`: the light class
 // takes it as given, the compute-heavy classes at most 2.
 constexpr int ClassIT(int c, int it) { return Base(c) == 0 ? it : (it < 2 ? it : 2); }
-// ... and 1 in a heavy class whose `items` queries would not give each CU
-// kHeavyTiles tiles: such a launch lasts as long as its longest lane, and a
+// ... and 1 in a heavy class whose `items` queries make fewer than kHeavyTiles
+// tiles (four a CU): such a launch lasts as long as its longest lane, and a
 // second item on that lane doubles it.
 constexpr uint64_t kHeavyTiles = 4 * 256;
 constexpr int RunIT(int c, int it, uint64_t items) {
